@@ -18,7 +18,9 @@
 //     schedule share one XCD's L2 (the weight panel is re-read from L2, not HBM).
 // Quantized path (codes of any width, 32x32 blocks, f32 W, N a multiple of 64): fp32 matrix
 // cores, bell_spmm_quant_mfma below.
-// Generic path (any other dtype / block size / N): one wave per row,
+// Unquantized values in blocks of 8, 16 or 32 against a row-major W of any type and width run on
+// the fp32 matrix cores, bell_spmm_plain_mfma below.
+// Generic path (any other block size, quantized shapes the above leave out): one wave per row,
 // lanes over output columns, slots in order, decoded with the codec exactly as
 // quantized_blocked_ell_spmm_fwd_kernel_ does
 // (src/compute/sparse/project/kernels/quantized_blocked_ell_spmm_fwd_kernel_.cuh:1-39).
@@ -1033,6 +1035,270 @@ __global__ __launch_bounds__(256) void bell_spmm_quant_lds(BellArgs a, std::int6
     }
 }
 
+// ---- unquantized values on the fp32 matrix cores -----------------------------------------
+//
+// Blocks of 8, 16 or 32, values and W of any type, any N (W row-major): every operand is
+// widened exactly to fp32 and multiplied on v_mfma_f32_16x16x4_f32 (fp32 products and sums;
+// only the summation order differs from bell_spmm_generic). One workgroup per (row block, 64
+// output columns); its waves take the row block's valid slots in turn (slot s to wave s modulo
+// the wave count) and their partial tiles are added pairwise through LDS at the end, in a fixed
+// order: a row block of one wave left most SIMDs idle on matrices of a few thousand rows.
+//
+// K runs permuted so that every lane loads whole vectors: at step kk lane group h = lane / 16
+// holds gene h * (bs / 4) + kk of the block in both operands, so A is one load of bs / 4
+// consecutive values per lane and slot (row lane % 16 of each 16-row tile). Columns run
+// permuted too: tile t of the four holds columns 4 (lane % 16) + t, so one 16-byte load of a
+// W row gives the lane its B operand of all four tiles, and a row's four results are one
+// 16-byte store. Blocks of 8 fill half of the 16 tile rows: the loads bound them, not the
+// matrix cores. The next slot's operands load while the current one's products run.
+//
+// Genes past `cols`, rows past the matrix and columns past N lie outside the loads' ranges and
+// read as 0 (values stored past `cols` are set to 0 too: NaN there must not reach the sums).
+//
+// Measured on 40,005 rows x 64 slots of 16 x 16 (48 valid on average), f16 values, f32 W,
+// N = 64: 47 us, 84 TFLOP/s of the 151 an fp32 library product reaches here; 2,657 us with
+// bell_spmm_generic (one load and one FMA per stored element and column, serial per row).
+
+enum WLoad : int { kWVec = 0, kWScalar = 1, kWHalf = 2 };  // f32 16 bytes a lane; f32; f16 or bf16
+
+template<int kValBytes, int kBs, int kW>
+struct PlainSlot {
+    static constexpr int kSteps = kBs / 4;
+    static constexpr int kTiles = kBs == 32 ? 2 : 1;
+    std::uint32_t a[kTiles][kSteps * kValBytes / 4];  // packed values of this lane's row(s)
+    float b[kSteps][4];
+    std::uint32_t genes;  // of the block below `cols`
+};
+
+template<int kValBytes, int kBs, int kW>
+__global__ __launch_bounds__(1024) void bell_spmm_plain_mfma(BellArgs a, std::uint32_t value_bf16,
+                                                             std::uint32_t rhs_bf16, std::uint32_t n,
+                                                             std::uint32_t chunks) {
+    using Slot = PlainSlot<kValBytes, kBs, kW>;
+    constexpr int kSteps = Slot::kSteps, kTiles = Slot::kTiles, kDw = kSteps * kValBytes / 4;
+    constexpr std::uint32_t kOut = 0x7ffffff0u;  // an offset outside every range (plain_applicable)
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    extern __shared__ float4 partial[];
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const std::uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const std::uint32_t waves = blockDim.x / kWave;  // a power of two
+    const std::uint32_t rb = blockIdx.x / chunks;
+    const std::uint32_t n0 = (blockIdx.x % chunks) * 64u;
+    const std::uint32_t width = a.ell_cols / kBs;
+    const std::uint32_t *slots = a.block_col_idx + static_cast<std::uint64_t>(rb) * width;
+    const std::uint32_t m = static_cast<std::uint32_t>(lane) % 16u, h = static_cast<std::uint32_t>(lane) / 16u;
+    const std::uint32_t block_rows = min(static_cast<std::uint32_t>(kBs), a.rows - rb * kBs);
+    const std::uint32_t row_pitch = a.ell_cols * kValBytes;
+    const rsrc_t ra = make_rsrc(static_cast<const char *>(a.values) + static_cast<std::uint64_t>(rb) * kBs * row_pitch,
+                                (a.block_major != 0u ? kBs : block_rows) * row_pitch);
+    std::uint32_t a_lane[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+        const std::uint32_t r = 16u * t + m;
+        a_lane[t] = r < block_rows ? r * a.a_row_bytes + h * kSteps * kValBytes : kOut;
+    }
+    constexpr std::uint32_t kWBytes = kW == kWHalf ? 2u : 4u;
+    const std::uint32_t w_pitch = static_cast<std::uint32_t>(a.rhs_ld) * kWBytes;
+    const std::uint32_t col = n0 + 4u * m;  // this lane's first column
+    const std::uint32_t live = col < n ? min(4u, n - col) : 0u;
+
+    auto load = [&](Slot &o, std::uint32_t s, std::uint32_t bc) {
+        const std::uint32_t so = s * a.a_slot_bytes;
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            const int off = static_cast<int>(a_lane[t] == kOut ? kOut : a_lane[t] + so);
+            if constexpr (kDw >= 4) {
+#pragma unroll
+                for (int q = 0; q < kDw / 4; ++q) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(ra, off + 16 * q, 0, 0);
+                    o.a[t][4 * q] = v[0]; o.a[t][4 * q + 1] = v[1]; o.a[t][4 * q + 2] = v[2]; o.a[t][4 * q + 3] = v[3];
+                }
+            } else if constexpr (kDw == 2) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(ra, off, 0, 0);
+                o.a[t][0] = v[0]; o.a[t][1] = v[1];
+            } else {
+                o.a[t][0] = static_cast<std::uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(ra, off, 0, 0));
+            }
+        }
+        const std::uint64_t g0 = static_cast<std::uint64_t>(bc) * kBs;
+        const std::uint32_t genes = g0 < a.cols ? min(static_cast<std::uint32_t>(kBs), a.cols - static_cast<std::uint32_t>(g0)) : 0u;
+        o.genes = genes;
+        const rsrc_t rw = make_rsrc(static_cast<const char *>(a.rhs) + (genes != 0u ? g0 : 0u) * w_pitch,
+                                    genes != 0u ? (genes - 1u) * w_pitch + n * kWBytes : 0u);
+#pragma unroll
+        for (int kk = 0; kk < kSteps; ++kk) {
+            const std::uint32_t off = (h * kSteps + kk) * w_pitch + col * kWBytes;
+            if constexpr (kW == kWVec) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, static_cast<int>(live != 0u ? off : kOut), 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) o.b[kk][t] = __uint_as_float(v[t]);
+            } else {
+#pragma unroll
+                for (std::uint32_t t = 0; t < 4u; ++t) {
+                    const int to = static_cast<int>(t < live ? off + t * kWBytes : kOut);
+                    if constexpr (kW == kWScalar) {
+                        o.b[kk][t] = __uint_as_float(static_cast<std::uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rw, to, 0, 0)));
+                    } else {
+                        const std::uint16_t bits = static_cast<std::uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rw, to, 0, 0));
+                        o.b[kk][t] = rhs_bf16 != 0u ? bf2f(bits) : h2f(bits);
+                    }
+                }
+            }
+        }
+    };
+    floatx4 acc[kTiles][4];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[t][q] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    auto multiply = [&](const Slot &o) {
+#pragma unroll
+        for (int kk = 0; kk < kSteps; ++kk) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) {
+                float x;
+                if constexpr (kValBytes == 4) {
+                    x = __uint_as_float(o.a[t][kk]);
+                } else {
+                    const std::uint16_t bits = static_cast<std::uint16_t>(o.a[t][kk / 2] >> (16 * (kk % 2)));
+                    x = value_bf16 != 0u ? bf2f(bits) : h2f(bits);
+                }
+                x = h * kSteps + kk < o.genes ? x : 0.0f;  // whatever is stored past `cols`
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[t][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, o.b[kk][q], acc[t][q], 0, 0, 0);
+            }
+        }
+    };
+
+    std::uint64_t mine = 1ull;  // this wave's slots of 64: wave, wave + waves, ...
+    for (std::uint32_t s = waves; s < 64u; s *= 2u) mine |= mine << s;
+    mine <<= wave;
+    for (std::uint32_t base = 0; base < width; base += kWave) {
+        const std::uint32_t sid = base + lane < width ? slots[base + lane] : kInvalidBlock;
+        std::uint64_t todo = __ballot(sid != kInvalidBlock) & mine;
+        if (todo == 0ull) continue;
+        auto next = [&](Slot &o) {
+            const int s = __builtin_ctzll(todo);
+            todo &= todo - 1ull;
+            load(o, base + s, static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(sid), s)));
+        };
+        Slot s0, s1;
+        next(s0);
+        for (;;) {  // two register sets in turn
+            if (todo != 0ull) next(s1);
+            else { multiply(s0); break; }
+            multiply(s0);
+            if (todo != 0ull) next(s0);
+            else { multiply(s1); break; }
+            multiply(s1);
+        }
+    }
+
+    // the waves' partial tiles, pairwise: wave w + half onto wave w
+    for (std::uint32_t half = waves / 2u; half != 0u; half /= 2u) {
+        if (wave >= half && wave < 2u * half) {
+            float4 *p = partial + (wave - half) * (kTiles * 4 * kWave) + lane;
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    p[(4 * t + q) * kWave] = make_float4(acc[t][q][0], acc[t][q][1], acc[t][q][2], acc[t][q][3]);
+        }
+        __syncthreads();
+        if (wave < half) {
+            const float4 *p = partial + wave * (kTiles * 4 * kWave) + lane;
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 v = p[(4 * t + q) * kWave];
+                    acc[t][q][0] += v.x; acc[t][q][1] += v.y; acc[t][q][2] += v.z; acc[t][q][3] += v.w;
+                }
+        }
+        __syncthreads();
+    }
+    if (wave != 0u) return;
+    // D layout: lane holds rows 4h + i of its tile; tile q is column col + q
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const std::uint32_t r = 16u * t + 4u * h + i;
+            if (r >= block_rows) continue;
+            const std::uint32_t row = rb * kBs + r;
+            float v[4];
+#pragma unroll
+            for (std::uint32_t q = 0; q < 4u; ++q)
+                v[q] = a.ep.active && q < live ? epilogue_value(a.ep, acc[t][q][i], row, col + q) : acc[t][q][i];
+            float *o = a.out + static_cast<std::int64_t>(row) * a.out_ld + col;
+            if constexpr (kW == kWVec) {
+                if (live != 0u) *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (std::uint32_t q = 0; q < 4u; ++q)
+                    if (q < live) o[q] = v[q];
+            }
+        }
+    }
+}
+
+// Waves per workgroup: enough that 256 CUs hold about four waves per SIMD, at most one per slot
+// (a power of two up to 16).
+std::uint32_t plain_waves(std::uint64_t groups, std::uint32_t width) {
+    std::uint32_t w = 4u;
+    while (w < 16u && groups * w < 4096u) w *= 2u;
+    while (w > 1u && w > width) w /= 2u;
+    return w;
+}
+
+template<int kValBytes, int kBs>
+void launch_plain(const BellArgs &a, std::uint32_t value_dtype, std::uint32_t rhs_dtype, std::uint32_t n, int w_mode,
+                  hipStream_t s) {
+    const std::uint32_t chunks = (n + 63u) / 64u, row_blocks = (a.rows + kBs - 1u) / kBs;
+    const std::uint32_t waves = plain_waves(static_cast<std::uint64_t>(row_blocks) * chunks, a.ell_cols / kBs);
+    const std::uint32_t lds = waves / 2u * (kBs == 32 ? 2u : 1u) * 4u * kWave * 16u;
+    const dim3 grid(row_blocks * chunks), block(waves * kWave);
+    const std::uint32_t vb = value_dtype == CELLERATOR_DTYPE_BF16, rb = rhs_dtype == CELLERATOR_DTYPE_BF16;
+    if (w_mode == kWVec)
+        hipLaunchKernelGGL((bell_spmm_plain_mfma<kValBytes, kBs, kWVec>), grid, block, lds, s, a, vb, rb, n, chunks);
+    else if (w_mode == kWScalar)
+        hipLaunchKernelGGL((bell_spmm_plain_mfma<kValBytes, kBs, kWScalar>), grid, block, lds, s, a, vb, rb, n, chunks);
+    else
+        hipLaunchKernelGGL((bell_spmm_plain_mfma<kValBytes, kBs, kWHalf>), grid, block, lds, s, a, vb, rb, n, chunks);
+}
+
+// The matrix-core form takes blocks of 8, 16 and 32 whose values start on 16 bytes and whose
+// ranges (a row block's values, a block column's W rows) fit 32-bit offsets; the rest keep
+// bell_spmm_generic.
+bool plain_applicable(const BellArgs &a, std::uint32_t value_dtype, std::uint32_t rhs_dtype, std::int64_t n) {
+    const std::uint64_t bs = a.block_size, vb = value_dtype == CELLERATOR_DTYPE_F32 ? 4u : 2u;
+    const std::uint64_t wb = rhs_dtype == CELLERATOR_DTYPE_F32 ? 4u : 2u;
+    constexpr std::uint64_t kRange = 0x7fff0000ull;
+    return (bs == 8u || bs == 16u || bs == 32u) && (reinterpret_cast<std::uintptr_t>(a.values) & 15u) == 0u
+        && (reinterpret_cast<std::uintptr_t>(a.rhs) & (wb - 1u)) == 0u
+        && bs * a.ell_cols * vb <= kRange && static_cast<std::uint64_t>(a.rhs_ld) <= kRange / (wb * bs)
+        && ((a.rows + bs - 1u) / bs) * ((static_cast<std::uint64_t>(n) + 63u) / 64u) <= kRange;
+}
+
+int launch_plain_bs(const BellArgs &a, std::uint32_t value_dtype, std::uint32_t rhs_dtype, std::int64_t n, hipStream_t s) {
+    const bool vec = (reinterpret_cast<std::uintptr_t>(a.rhs) & 15u) == 0u && a.rhs_ld % 4 == 0 && n % 4 == 0
+        && (reinterpret_cast<std::uintptr_t>(a.out) & 15u) == 0u && a.out_ld % 4 == 0;
+    const int mode = rhs_dtype != CELLERATOR_DTYPE_F32 ? kWHalf : vec ? kWVec : kWScalar;
+    const std::uint32_t nn = static_cast<std::uint32_t>(n);
+    if (value_dtype == CELLERATOR_DTYPE_F32) {
+        if (a.block_size == 8u) launch_plain<4, 8>(a, value_dtype, rhs_dtype, nn, mode, s);
+        else if (a.block_size == 16u) launch_plain<4, 16>(a, value_dtype, rhs_dtype, nn, mode, s);
+        else launch_plain<4, 32>(a, value_dtype, rhs_dtype, nn, mode, s);
+    } else {
+        if (a.block_size == 8u) launch_plain<2, 8>(a, value_dtype, rhs_dtype, nn, mode, s);
+        else if (a.block_size == 16u) launch_plain<2, 16>(a, value_dtype, rhs_dtype, nn, mode, s);
+        else launch_plain<2, 32>(a, value_dtype, rhs_dtype, nn, mode, s);
+    }
+    return check_launch("bell_spmm_plain_mfma");
+}
+
 int validate_bell(const cx_bell_matrix *m, const void *rhs, std::int64_t rhs_ld,
                   std::int64_t out_cols, const float *out, std::int64_t out_ld) {
     if (m == nullptr || rhs == nullptr || out == nullptr)
@@ -1177,6 +1443,8 @@ int bell_spmm_fwd_impl(const cx_bell_matrix *m, const void *rhs, uint32_t rhs_dt
 #undef CX_QBELL_W
         return check_launch("bell_spmm_quant_mfma");
     }
+    if (m->bits == 0u && plain_applicable(a, m->value_dtype, rhs_dtype, out_cols))
+        return launch_plain_bs(a, m->value_dtype, rhs_dtype, out_cols, static_cast<hipStream_t>(stream));
     // the per-element kernel walks rows in matrix order (no row-block order)
     const std::uint64_t threads = static_cast<std::uint64_t>(m->rows) * kWave;
     hipLaunchKernelGGL(bell_spmm_generic, dim3(static_cast<unsigned>((threads + 255) / 256)),

@@ -1,0 +1,56 @@
+"""Blocked-ELL with unquantized values on the fp32 matrix cores (bell_spmm_plain_mfma): the edges
+of its tiles and of its dispatch against the float64 referee."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.helpers import check_against_referee
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("value_dtype,rhs_dtype", [("float16", "float32"), ("float32", "float32"),
+                                                   ("bfloat16", "float16"), ("float32", "bfloat16")])
+@pytest.mark.parametrize("rows,n,width,pad", [(1, 1, 1, 0), (67, 50, 5, 0), (200, 64, 70, 0), (96, 100, 3, 4),
+                                              (33, 130, 17, 1), (1200, 128, 9, 8)])
+def test_plain_bell_edges(oracle, bs, value_dtype, rhs_dtype, rows, n, width, pad):
+    """Ragged last row block and block column, slot lists from one to more than a wave's lanes,
+    invalid slots anywhere, NaN in every value that must not be read into a sum, W rows of N + pad
+    (16-byte rows and not), both value layouts, and the bias + ReLU store."""
+    import torch
+
+    from cellerator_amd import BellMatrix, Epilogue, bell_block_major, bell_spmm
+    from cellerator_amd import _native as N
+    rng = np.random.default_rng(bs * 1000 + rows + n)
+    cols = 7 * bs + 3
+    rb, kb = -(-rows // bs), -(-cols // bs)
+    idx = rng.integers(0, kb, (rb, width)).astype(np.uint32)
+    idx[rng.random((rb, width)) < 0.3] = 0xFFFFFFFF
+    vd, wd = getattr(torch, value_dtype), getattr(torch, rhs_dtype)
+    vals = torch.from_numpy(rng.standard_normal((rows, width * bs)).astype(np.float32)).to(vd)
+    gene = np.where(idx == 0xFFFFFFFF, cols, idx).repeat(bs, axis=1).astype(np.int64) * bs + np.tile(np.arange(bs), width)
+    dead = torch.from_numpy(np.repeat(gene >= cols, bs, axis=0)[:rows])
+    w = torch.from_numpy(rng.standard_normal((cols, n + pad)).astype(np.float32)).to(wd)
+    clean = torch.where(dead, torch.zeros_like(vals), vals)
+    vals = torch.where(dead, torch.full_like(vals, float("nan")), vals)
+    # the referee takes exact fp32 copies of the widened operands
+    full = np.zeros((rb * bs, width * bs), np.float32)
+    full[:rows] = clean.float().numpy()
+    ref, mag = oracle.bell_spmm_referee(rows, cols, bs, width * bs, idx, full, w[:, :n].float().contiguous().numpy(),
+                                        value_type=oracle.F32)
+    m = BellMatrix(rows, cols, bs, width * bs, torch.from_numpy(idx.view(np.int32)).cuda(), values=vals.cuda())
+    wg = w.cuda()[:, :n]
+    out = bell_spmm(m, wg)
+    assert torch.isfinite(out).all()
+    check_against_referee(oracle, ref, mag, out.cpu().numpy())
+    assert torch.equal(out, bell_spmm(bell_block_major(m), wg))
+    bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
+    assert torch.equal(bell_spmm(m, wg, epilogue=Epilogue(kind=N.EPILOGUE_BIAS_RELU, bias=bias)),
+                       torch.relu(out + bias))
+    # W and Y off a 16-byte boundary (the same sums, single-column loads)
+    if rhs_dtype == "float32":
+        shifted = torch.empty(cols * (n + pad) + 1, device="cuda")[1:].view(cols, n + pad)
+        shifted.copy_(w.cuda())
+        assert torch.equal(out, bell_spmm(m, shifted[:, :n]))
