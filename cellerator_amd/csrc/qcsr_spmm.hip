@@ -18,10 +18,15 @@
 //     (v_fma_mix_f32 for fp16 weights: widening folded into the FMA);
 //   * at the end of the row the kEps group partials are summed with a xor butterfly
 //     and group 0 writes the row's N outputs (one 16/32 B store per lane).
+// qcsr_spmm_split is that form for every plain launch (a row to 1 .. 16 waves, so a few hundred
+// cells fill the chip); qcsr_spmm_rowwave stays for weights past its 2 GiB descriptor and the
+// load-balanced form cuts equal entry ranges. Quantized codes with fp16 weights at N = 64 .. 256
+// leave for the row groups of qcsr_parts.hip above split_preferred's line.
 // Any other shape (N not 32/64/128, unaligned operands) takes the generic kernel: one
 // wave per row, lanes over output columns, entries in nnz order.
 #include "qcsr_common.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace cx {
@@ -147,6 +152,147 @@ __global__ __launch_bounds__(kWave *kWavesPerBlock) void qcsr_spmm_rowwave(QcsrA
     accumulate_segment<kBits, kPolicy, kMode, RhsT, kN>(a, stage[wave], row, begin, begin, end, lane, acc);
     reduce_groups<S::kLpe, S::kCpl>(acc);
     if (lane < S::kLpe) store_row<S::kCpl>(a, row, lane, acc);
+}
+
+// ---- split rows: 1 to 16 waves per row ---------------------------------------------------
+
+// Byte offset of a staged entry that reads as 0: past every W range (split_applicable).
+constexpr std::uint32_t kNoEntry = 0x7fff8000u;
+
+// The row-wave form with each row's 64-entry chunks dealt to 2^log_split waves of a workgroup
+// (chunk c to wave c modulo their count) whose sums are added through LDS in wave order. The
+// next chunk's columns and codes load under the current chunk's weight gathers, and W rows are
+// read at 32-bit offsets through a buffer descriptor over exactly [cols x N], so an entry whose
+// column lies outside [0, cols), or past the chunk's end, reads zeros and adds nothing.
+template<int kBits, int kPolicy, ValueMode kMode, typename RhsT, int kN>
+__global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int log_split) {
+    using S = WaveShape<RhsT, kN>;
+    constexpr int kCpl = S::kCpl, kLpe = S::kLpe, kEps = S::kEps;
+    constexpr int kBatch = 4;  // steps whose gathers are in flight together
+    __shared__ uint2 stage_all[16][kWave];
+    __shared__ float part[16][kN];
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const int sub = wave & ((1 << log_split) - 1);
+    const std::uint32_t row = blockIdx.x * ((blockDim.x / kWave) >> log_split) + (wave >> log_split);
+    const int g = lane / kLpe;
+    const int j = lane % kLpe;
+    uint2 *stage = stage_all[wave];
+    const std::uint32_t row_bytes = static_cast<std::uint32_t>(a.rhs_ld) * sizeof(RhsT);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<void *>(a.rhs), static_cast<short>(0),
+        a.cols != 0u ? static_cast<int>((a.cols - 1u) * row_bytes + kN * sizeof(RhsT)) : 0, 0x00020000);
+    float acc[kCpl];
+#pragma unroll
+    for (int k = 0; k < kCpl; ++k) acc[k] = 0.0f;
+
+    if (row < a.rows) {
+        const std::uint32_t begin = static_cast<std::uint32_t>(a.row_ptr[row]);
+        const std::uint32_t end = static_cast<std::uint32_t>(a.row_ptr[row + 1]);
+        const std::uint8_t *pbase = nullptr;
+        float row_offset = 0.0f;
+        if constexpr (kMode == ValueMode::quantized) {
+            pbase = a.packed + a.packed_row_ptr[row];
+            if constexpr (kPolicy == CX_DECODE_COLUMN_SCALE_ROW_OFFSET)
+                row_offset = a.row_offsets != nullptr ? a.row_offsets[row] : 0.0f;
+        }
+        // a lane's entry as stored: its column (-1 past the row) and its code byte or value
+        struct Raw {
+            std::int32_t col;
+            std::uint32_t bits;
+        };
+        auto load_raw = [&](std::uint32_t c0) {
+            Raw r{-1, 0u};
+            const std::uint32_t i = c0 + lane;
+            if (i < end) {
+                r.col = a.col_idx[i];
+                if constexpr (kMode == ValueMode::quantized) r.bits = pbase[(i - begin) / (8 / kBits)];
+                else if constexpr (kMode == ValueMode::f16) r.bits = static_cast<const std::uint16_t *>(a.values)[i];
+                else r.bits = static_cast<const std::uint32_t *>(a.values)[i];
+            }
+            return r;
+        };
+        const std::uint32_t step = static_cast<std::uint32_t>(kWave) << log_split;
+        std::uint32_t c0 = begin + sub * kWave;
+        Raw cur = load_raw(c0);
+        for (; c0 < end; c0 += step) {
+            const bool ok = static_cast<std::uint32_t>(cur.col) < a.cols;
+            float x = 0.0f;
+            if constexpr (kMode == ValueMode::quantized) {
+                float2 md = make_float2(0.0f, 0.0f);
+                if constexpr (kPolicy == CX_DECODE_PER_GENE_AFFINE_PAIRS) {
+                    if (ok) md = reinterpret_cast<const float2 *>(a.scales)[cur.col];
+                } else if (ok) {
+                    md.x = a.scales != nullptr ? a.scales[cur.col] : 1.0f;
+                    md.y = kPolicy == CX_DECODE_PER_GENE_AFFINE ? (a.offsets != nullptr ? a.offsets[cur.col] : 0.0f)
+                                                                : row_offset;
+                }
+                constexpr std::uint32_t kCpb = 8 / kBits;
+                const std::uint32_t shift = (c0 + lane - begin) % kCpb * kBits;
+                const std::uint32_t code = (cur.bits >> shift) & ((1u << kBits) - 1u);
+                x = __builtin_fmaf(static_cast<float>(code), md.x, md.y);
+            } else if constexpr (kMode == ValueMode::f16) {
+                x = h2f(static_cast<std::uint16_t>(cur.bits));
+            } else {
+                x = __uint_as_float(cur.bits);
+            }
+            stage[lane] = make_uint2(ok ? static_cast<std::uint32_t>(cur.col) * row_bytes : kNoEntry,
+                                     ok ? __float_as_uint(x) : 0u);
+            wave_sync();
+            const int count = static_cast<int>(min(end - c0, static_cast<std::uint32_t>(kWave)));
+            cur = load_raw(c0 + step);
+            for (int s0 = 0; s0 < count; s0 += kBatch * kEps) {
+                uint2 e[kBatch];
+                float4 w[kBatch];
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q) {
+                    e[q] = stage[s0 + q * kEps + g];
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, static_cast<int>(e[q].x + j * 16u), 0, 0);
+                    w[q] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+                }
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q)
+                    fma_row<RhsT, kCpl>(acc, __uint_as_float(e[q].y), reinterpret_cast<const RhsT *>(&w[q]));
+            }
+            wave_sync();
+        }
+        reduce_groups<kLpe, kCpl>(acc);
+    }
+    if (log_split == 0) {
+        if (row < a.rows && lane < kLpe) store_row<kCpl>(a, row, lane, acc);
+        return;
+    }
+    if (lane < kLpe) {
+#pragma unroll
+        for (int k = 0; k < kCpl; ++k) part[wave][lane * kCpl + k] = acc[k];
+    }
+    __syncthreads();
+    if (sub != 0 || row >= a.rows) return;
+    for (int c = lane; c < kN; c += kWave) {
+        float v = part[wave][c];
+        for (int q = 1; q < (1 << log_split); ++q) v += part[wave + q][c];
+        a.out[static_cast<std::int64_t>(row) * a.out_ld + c] = a.ep.active ? epilogue_value(a.ep, v, row, c) : v;
+    }
+}
+
+// W read at 32-bit offsets below kNoEntry.
+bool split_applicable(const QcsrArgs &a, std::size_t esize, std::int64_t n) {
+    return static_cast<std::uint64_t>(a.cols) * static_cast<std::uint64_t>(a.rhs_ld) * esize + n * esize <= 0x7fff0000ull;
+}
+
+// Waves per row (log2): about 8 waves per SIMD over the chip, and at least one chunk per wave.
+int split_log(const QcsrArgs &a, std::uint64_t nnz) {
+    int l = 0;
+    while (l < 4 && (static_cast<std::uint64_t>(a.rows) << l) < 8192u && (nnz / a.rows) >> l > kWave) ++l;
+    return l;
+}
+
+template<int kBits, int kPolicy, ValueMode kMode, typename RhsT, int kN>
+void launch_split(const QcsrArgs &a, int log_split, hipStream_t stream) {
+    const int waves = log_split <= 2 ? 4 : 1 << log_split;
+    const std::uint32_t rows_per_block = static_cast<std::uint32_t>(waves >> log_split);
+    hipLaunchKernelGGL((qcsr_spmm_split<kBits, kPolicy, kMode, RhsT, kN>),
+                       dim3((a.rows + rows_per_block - 1u) / rows_per_block), dim3(waves * kWave), 0, stream, a, log_split);
 }
 
 // ---- load-balanced form: equal nnz chunks, one wave per chunk ----------------------------
@@ -282,7 +428,7 @@ int launch_balanced(const QcsrArgs &a, const Balance &b, hipStream_t stream) {
 }
 
 template<int kBits, int kPolicy, ValueMode kMode, typename RhsT>
-int launch_rhs(const QcsrArgs &a, std::int64_t n, bool aligned, const Balance *bal,
+int launch_rhs(const QcsrArgs &a, std::int64_t n, bool aligned, const Balance *bal, std::uint64_t nnz,
                hipStream_t stream) {
     const unsigned blocks = (a.rows + kWavesPerBlock - 1) / kWavesPerBlock;
     const dim3 grid(blocks), block(kWave * kWavesPerBlock);
@@ -291,7 +437,12 @@ int launch_rhs(const QcsrArgs &a, std::int64_t n, bool aligned, const Balance *b
         return launch_balanced<kBits, kPolicy, kMode, RhsT, 64>(a, *bal, stream);
     if (bal != nullptr && aligned && n == 128)
         return launch_balanced<kBits, kPolicy, kMode, RhsT, 128>(a, *bal, stream);
-    if (aligned && n == 64) {
+    if (aligned && (n == 32 || n == 64 || n == 128) && split_applicable(a, sizeof(RhsT), n)) {
+        const int l = split_log(a, nnz);
+        if (n == 32) launch_split<kBits, kPolicy, kMode, RhsT, 32>(a, l, stream);
+        else if (n == 64) launch_split<kBits, kPolicy, kMode, RhsT, 64>(a, l, stream);
+        else launch_split<kBits, kPolicy, kMode, RhsT, 128>(a, l, stream);
+    } else if (aligned && n == 64) {
         hipLaunchKernelGGL((qcsr_spmm_rowwave<kBits, kPolicy, kMode, RhsT, 64>), grid, block, 0,
                            stream, a);
     } else if (aligned && n == 128) {
@@ -309,22 +460,48 @@ int launch_rhs(const QcsrArgs &a, std::int64_t n, bool aligned, const Balance *b
 
 template<int kBits, int kPolicy, ValueMode kMode>
 int launch_mode(const QcsrArgs &a, std::uint32_t rhs_dtype, std::int64_t n, bool aligned,
-                const Balance *bal, hipStream_t stream) {
+                const Balance *bal, std::uint64_t nnz, hipStream_t stream) {
     if (rhs_dtype == CELLERATOR_DTYPE_F16)
-        return launch_rhs<kBits, kPolicy, kMode, std::uint16_t>(a, n, aligned, bal, stream);
-    return launch_rhs<kBits, kPolicy, kMode, float>(a, n, aligned, bal, stream);
+        return launch_rhs<kBits, kPolicy, kMode, std::uint16_t>(a, n, aligned, bal, nnz, stream);
+    return launch_rhs<kBits, kPolicy, kMode, float>(a, n, aligned, bal, nnz, stream);
 }
 
 template<int kPolicy>
 int launch_bits(const QcsrArgs &a, std::uint32_t bits, std::uint32_t rhs_dtype, std::int64_t n,
-                bool aligned, const Balance *bal, hipStream_t stream) {
+                bool aligned, const Balance *bal, std::uint64_t nnz, hipStream_t stream) {
     switch (bits) {
-    case 1: return launch_mode<1, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, stream);
-    case 2: return launch_mode<2, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, stream);
-    case 4: return launch_mode<4, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, stream);
-    case 8: return launch_mode<8, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, stream);
+    case 1: return launch_mode<1, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, nnz, stream);
+    case 2: return launch_mode<2, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, nnz, stream);
+    case 4: return launch_mode<4, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, nnz, stream);
+    case 8: return launch_mode<8, kPolicy, ValueMode::quantized>(a, rhs_dtype, n, aligned, bal, nnz, stream);
     default: return fail(CX_STATUS_UNSUPPORTED, "quantized CSR bits must be 1, 2, 4 or 8");
     }
+}
+
+int launch_quantized(const QcsrArgs &a, const cx_qcsr_matrix &m, std::uint32_t rhs_dtype, std::int64_t n, bool aligned,
+                     const Balance *bal, hipStream_t s) {
+    if (m.decode_policy == CX_DECODE_PER_GENE_AFFINE)
+        return launch_bits<CX_DECODE_PER_GENE_AFFINE>(a, m.bits, rhs_dtype, n, aligned, bal, m.nnz, s);
+    if (m.decode_policy == CX_DECODE_PER_GENE_AFFINE_PAIRS)
+        return launch_bits<CX_DECODE_PER_GENE_AFFINE_PAIRS>(a, m.bits, rhs_dtype, n, aligned, bal, m.nnz, s);
+    return launch_bits<CX_DECODE_COLUMN_SCALE_ROW_OFFSET>(a, m.bits, rhs_dtype, n, aligned, bal, m.nnz, s);
+}
+
+// Where the split rows beat the row groups over LDS gene parts (qcsr_parts.hip), for the shapes
+// both take. The split rows' time is their gathers', about 10 us per million entries for 64
+// output columns and 17 for 128 (the columns and codes are read once); the row groups pay for
+// walking every gene part with few rows per workgroup before the entries count. Times in us,
+// split / row groups, by rows (33,538 genes of 1,500 per row; 33,538 of 300; 4,000 of 300):
+//   N = 64:    250: 12 / 359, 11 / 158, 9 / 82;   30,000: 474 / 643, 105 / 223, 80 / 143;
+//           60,000: 1,101 / 996, 204 / 295, 154 / 214;  120,000: 1,829 / 1,049, 331 / 370, 248 / 229
+//   N = 128: 30,000: 845 / 1,284, 174 / 440, 132 / 281; 120,000: 2,982 / 2,079, 536 / 738, 418 / 448
+// So the line is drawn at 30 million entries plus one million per gene part, half as far
+// again where the output is whole blocks of 128 columns.
+bool split_preferred(const QcsrArgs &a, std::uint64_t nnz, std::int64_t n) {
+    const std::uint64_t parts = (a.cols + 1023u) / 1024u;
+    std::uint64_t line = 30'000'000u + parts * 1'000'000u;
+    if (n % 128 == 0) line += line / 2u;
+    return nnz < line && split_applicable(a, sizeof(std::uint16_t), n);
 }
 
 __global__ void pack_gene_affine_kernel(const float *scales, const float *offsets, std::uint32_t cols,
@@ -473,21 +650,28 @@ int qcsr_forward(const cx_qcsr_matrix *m, const void *rhs, std::uint32_t rhs_dty
         balance.chunks = static_cast<std::uint32_t>((m->nnz + balance.chunk - 1u) / balance.chunk);
         bal = &balance;
     }
-    if (bal == nullptr && qcsr_parts_applicable(a, m->bits, rhs_dtype, out_cols, aligned))
-        return launch_qcsr_parts(a, m->bits, m->decode_policy, out_cols, s);
+    if (bal == nullptr && qcsr_parts_applicable(a, m->bits, rhs_dtype, out_cols, aligned)) {
+        if (!split_preferred(a, m->nnz, out_cols)) return launch_qcsr_parts(a, m->bits, m->decode_policy, out_cols, s);
+        // the split rows in blocks of 128 output columns and a last one of 64
+        for (std::int64_t c0 = 0; c0 < out_cols; c0 += 128) {
+            QcsrArgs b = a;
+            b.rhs = static_cast<const std::uint16_t *>(a.rhs) + c0;
+            b.out = a.out + c0;
+            if (b.ep.bias != nullptr) b.ep.bias += c0;
+            if (b.ep.initial != nullptr) b.ep.initial += c0;
+            const int rc = launch_quantized(b, *m, rhs_dtype, std::min<std::int64_t>(128, out_cols - c0), aligned, nullptr, s);
+            if (rc != CX_STATUS_SUCCESS) return rc;
+        }
+        return CX_STATUS_SUCCESS;
+    }
     if (m->bits == 0u) {
         if (m->value_dtype == CELLERATOR_DTYPE_F16)
             return launch_mode<0, CX_DECODE_PER_GENE_AFFINE, ValueMode::f16>(a, rhs_dtype,
-                                                                               out_cols, aligned, bal, s);
+                                                                               out_cols, aligned, bal, m->nnz, s);
         return launch_mode<0, CX_DECODE_PER_GENE_AFFINE, ValueMode::f32>(a, rhs_dtype, out_cols,
-                                                                          aligned, bal, s);
+                                                                          aligned, bal, m->nnz, s);
     }
-    if (m->decode_policy == CX_DECODE_PER_GENE_AFFINE)
-        return launch_bits<CX_DECODE_PER_GENE_AFFINE>(a, m->bits, rhs_dtype, out_cols, aligned, bal, s);
-    if (m->decode_policy == CX_DECODE_PER_GENE_AFFINE_PAIRS)
-        return launch_bits<CX_DECODE_PER_GENE_AFFINE_PAIRS>(a, m->bits, rhs_dtype, out_cols, aligned, bal, s);
-    return launch_bits<CX_DECODE_COLUMN_SCALE_ROW_OFFSET>(a, m->bits, rhs_dtype, out_cols, aligned,
-                                                          bal, s);
+    return launch_quantized(a, *m, rhs_dtype, out_cols, aligned, bal, s);
 }
 
 } // namespace

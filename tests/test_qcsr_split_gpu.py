@@ -1,0 +1,77 @@
+"""The split-row quantized CSR SpMM (qcsr_spmm_split) at the edges of its shapes, and the row
+groups on a matrix large enough that the dispatch still takes them."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.helpers import check_against_referee, quantized_fixture, to_device_qcsr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits,policy", [(1, 2), (2, 1), (4, 1), (8, 2)])
+@pytest.mark.parametrize("rows,mean,n,dtype", [(1, 900.0, 64, np.float16), (3, 2500.0, 128, np.float16),
+                                               (9, 70.0, 256, np.float16), (37, 130.0, 192, np.float16),
+                                               (600, 64.0, 64, np.float32), (70, 300.0, 32, np.float32),
+                                               (33, 200.0, 128, np.float32), (2100, 33.0, 32, np.float16)])
+def test_split_rows(oracle, bits, policy, rows, mean, n, dtype):
+    """One to sixteen waves per row, empty rows, every lane split of W, blocks of 128 and 64
+    output columns, and columns outside [0, cols), which add nothing even when W holds
+    infinities."""
+    import torch
+
+    from cellerator_amd import Epilogue, qcsr_spmm
+    from cellerator_amd import _native as N
+    rng = np.random.default_rng(rows * 10 + bits + n)
+    fx = quantized_fixture(oracle, rng, rows, 3000, mean, bits, policy, empty_every=0 if rows == 1 else 4)
+    w = (rng.standard_normal((3000, n)) * 0.02).astype(dtype)
+    ref, mag = oracle.qcsr_spmm_referee(bits, policy, rows, 3000, fx["row_ptr"], fx["packed_row_ptr"], fx["col_idx"],
+                                        fx["packed"], fx["scales"], fx["offsets"], fx["row_offsets"], w)
+    m = to_device_qcsr(fx)
+    wt = torch.from_numpy(w).cuda()
+    out = qcsr_spmm(m, wt)
+    check_against_referee(oracle, ref, mag, out.cpu().numpy())
+    bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
+    got = qcsr_spmm(m, wt, epilogue=Epilogue(kind=N.EPILOGUE_BIAS_RELU, bias=bias))
+    assert torch.equal(got, torch.relu(out + bias))
+    # entries pointing outside the matrix: the row's other entries alone, with W[0] infinite
+    if len(fx["col_idx"]) > 2 and not (fx["col_idx"] == 0).any():
+        bad = np.random.default_rng(1).choice(len(fx["col_idx"]), size=max(1, len(fx["col_idx"]) // 9), replace=False)
+        col = m.col_idx.clone()
+        col[torch.from_numpy(bad).cuda()] = torch.tensor([-1, 3000, 2**31 - 1], dtype=torch.int32, device="cuda")[
+            torch.arange(len(bad), device="cuda") % 3]
+        m.col_idx = col
+        wt[0] = float("inf")
+        assert torch.isfinite(qcsr_spmm(m, wt)).all()
+
+
+@pytest.mark.parametrize("bits,policy,n", [(4, 3, 64), (8, 1, 64), (2, 2, 128)])
+def test_row_groups_above_the_line(bits, policy, n):
+    """A matrix past split_preferred's line runs on the row groups: a sample of rows from every
+    part of it against float64 (the bound of tests/helpers.py)."""
+    import torch
+
+    from cellerator_amd import QcsrMatrix, qcsr_check_columns, qcsr_pack_gene_affine, qcsr_spmm
+    from cellerator_amd import _native as N
+    from cellerator_amd.synth import QcsrConfig, dense_normal, generate_qcsr
+    rows, cols = 72_000, 6_000
+    m = generate_qcsr(QcsrConfig("line", rows, cols, bits, 1_000.0, 0.4, zipf_s=0.6, seed=5 + bits))
+    assert m.nnz > (30_000_000 + 6_000_000) * (1.5 if n == 128 else 1.0)
+    w = dense_normal((cols, n), 0.02, torch.float16, seed=3)
+    if policy == 2:
+        m = QcsrMatrix(rows, cols, bits, m.row_ptr, m.col_idx, packed_row_ptr=m.packed_row_ptr,
+                       packed_values=m.packed_values, column_scales=m.column_scales,
+                       row_offsets=torch.rand(rows, device="cuda"), decode_policy=N.DECODE_COLUMN_SCALE_ROW_OFFSET)
+    y = qcsr_spmm(qcsr_check_columns(qcsr_pack_gene_affine(m) if policy == 3 else m), w)
+    for r in list(range(0, 40)) + list(range(35_000, 35_040)) + list(range(rows - 40, rows)):
+        b, e = int(m.row_ptr[r]), int(m.row_ptr[r + 1])
+        i = torch.arange(e - b, device="cuda")
+        cpb = 8 // bits
+        byte = m.packed_values[int(m.packed_row_ptr[r]) + i // cpb].long()
+        code = ((byte >> ((i % cpb) * bits)) & ((1 << bits) - 1)).double()
+        c = m.col_idx[b:e].long()
+        off = m.row_offsets[r].double() if policy == 2 else m.column_offsets.double()[c]
+        x = code * m.column_scales.double()[c] + off
+        ref, mag = x @ w.double()[c], x.abs() @ w.double()[c].abs()
+        assert ((y[r].double() - ref).abs() <= 1e-4 * ref.abs() + 2.0 ** -20 * mag).all(), r
