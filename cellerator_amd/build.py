@@ -38,6 +38,7 @@ ENGINE_SOURCES = [
     "bell_spmm.hip",
     "cpbp_reduce.hip",
     "csr_spmv.hip",
+    "csr_parts.hip",
     "abi.cpp",
     "cpbp_build.cpp",
     "cpbp_build_device.hip",

@@ -1,0 +1,427 @@
+// csr_parts.hip -- Y = A . G for an unquantized f32 CSR and f32 G, with G streamed through LDS in
+// parts of 512 rows: the backward's grad_rhs = A^T . G (genes x cells, cells x N).
+//
+// Why: gathering a 256-byte row of G per entry through the texture path costs 4 cycles per entry
+// and CU at its 64 bytes a cycle whatever the caches hold. LDS serves the same rows in about 1.5,
+// and a row of 64 fp32 values is exactly 16 lanes x 16 bytes, so an entry can be handed round
+// by DPP instead of through a stage in LDS:
+//   * a group of 16 lanes (a DPP row) owns one row of A in each of the wave's kLayers layers and
+//     lane i holds its columns 4i .. 4i + 3; a wave works on 4 rows at a time;
+//   * lane i of the group loads entry i of the row's next 16; entries of the current part (a
+//     prefix: the columns ascend) turn into the LDS offset of their G row, the rest into an
+//     all-zero row and value 0;
+//   * step n broadcasts the group's n-th entry in the operand itself (row_newbcast): one
+//     v_add_u32_dpp (offset), one ds_read_b128 and four v_fmac_f32_dpp serve four entries.
+//
+// Rows are taken in order of length (a counting sort, once per call): the four rows of a layer
+// have similar runs, and the layers are dealt to the waves in snake order, so the waves of a
+// workgroup reach the barrier of each part together. A workgroup owns a set of 16 waves'
+// rows and a range of parts; long sets are cut into more ranges, so every workgroup carries
+// about the same work. A row's sum is taken part by part (a fresh sum of at most 512 terms per
+// part), then over the parts of its range, then over the ranges in order: fixed, and closer to
+// 64 bits than one chain over thousands of entries.
+//
+// Rows whose columns do not ascend through the parts (the walk would leave entries behind) are
+// found by it and summed again entry by entry in the last kernel; columns outside [0, cols)
+// add nothing there.
+//
+// Measured on the transpose of 100k cells x 20,000 genes, 200M entries, N = 64: 1,247 us (walk
+// 1,184, plan 32, ranges added up 32) against 6,050 with the balanced gathers; error against 64
+// bits 2.8e-7 against 4.7e-7.
+#include "qcsr_common.hpp"
+
+#include <algorithm>
+
+namespace cx {
+namespace {
+
+constexpr int kCells = 512;                       // G rows per part: 128 KB of LDS
+constexpr int kWaves = 16;
+constexpr int kLayers = 10;                       // 11 and 12 spill
+constexpr int kSetRows = kWaves * kLayers * 4;    // 640
+constexpr std::uint32_t kNone = 0xffffffffu;
+constexpr std::uint32_t kZeroRow = kCells * 256u;  // LDS offset of the all-zero row
+constexpr int kBuckets = 1024;                    // row lengths, 5 bits of mantissa
+constexpr std::uint32_t kMaxRows = 1u << 18;
+// What a part costs a workgroup besides its entries (the copy, two barriers, and a visit to
+// every layer), in entries: about 15k cycles at 1.25 cycles per entry.
+constexpr std::uint32_t kPartEntries = 12'000;
+
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+using lds_ptr = __attribute__((address_space(3))) void *;
+
+struct Item {
+    std::uint32_t set, part0, part1, split;  // set = kNone: nothing to do
+};
+
+struct Plan {
+    std::uint32_t *order;      // [sets * kSetRows] row of (set, wave, layer, group)
+    std::uint32_t *row_slot;   // [rows] its place in `order`
+    std::uint32_t *broken;     // [rows] nonzero: the walk could not finish it
+    std::uint32_t *splits;     // [sets] ranges of the set
+    std::uint32_t *first;      // [sets] its first item
+    Item *items;               // [max_items]
+    float *partials;           // [max_items][kSetRows][64]
+    std::uint32_t sets, max_items, parts;
+};
+
+// Longer rows first: 1,023 - (exponent, 5 bits of mantissa); 0 entries last.
+__device__ __forceinline__ std::uint32_t bucket_of(std::uint32_t len) {
+    if (len == 0u) return kBuckets - 1;
+    const std::uint32_t e = 31u - static_cast<std::uint32_t>(__builtin_clz(len));
+    const std::uint32_t m = (len << (31u - e)) >> 26 & 31u;
+    return kBuckets - 2u - min(e * 32u + m, kBuckets - 2u);
+}
+
+// Slot of the p-th longest row: quads of 4 rows, dealt to the waves of all sets in snake order,
+// 16 neighbouring waves to a set.
+__device__ __forceinline__ std::uint32_t slot_of(std::uint32_t p, std::uint32_t waves) {
+    const std::uint32_t quad = p / 4u, layer = quad / waves, at = quad % waves;
+    const std::uint32_t w = layer % 2u == 0u ? at : waves - 1u - at;
+    return (w * kLayers + layer) * 4u + p % 4u;
+}
+
+// One workgroup: the order of the rows, and the sets' ranges.
+__global__ __launch_bounds__(1024) void csr_parts_plan(const std::int32_t *row_ptr, std::uint32_t rows, Plan p) {
+    __shared__ std::uint32_t at[kBuckets];
+    __shared__ std::uint32_t scan[1024];
+    __shared__ std::uint32_t load[kMaxRows / kSetRows + 2];
+    const std::uint32_t tid = threadIdx.x;
+    at[tid] = 0u;
+    for (std::uint32_t s = tid; s < p.sets; s += 1024u) load[s] = 0u;
+    for (std::uint32_t i = rows + tid; i < p.sets * kSetRows; i += 1024u) p.order[slot_of(i, p.sets * kWaves)] = kNone;
+    __syncthreads();
+    for (std::uint32_t r0 = tid; r0 < rows; r0 += 4096u) {
+#pragma unroll
+        for (std::uint32_t k = 0; k < 4u; ++k) {
+            const std::uint32_t r = r0 + 1024u * k;
+            if (r >= rows) continue;
+            p.broken[r] = 0u;
+            const int len = row_ptr[r + 1] - row_ptr[r];
+            atomicAdd(&at[bucket_of(len > 0 ? static_cast<std::uint32_t>(len) : 0u)], 1u);
+        }
+    }
+    __syncthreads();
+    auto exclusive = [&](std::uint32_t v) {  // over the 1,024 threads
+        scan[tid] = v;
+        __syncthreads();
+        for (std::uint32_t d = 1u; d < 1024u; d *= 2u) {
+            const std::uint32_t u = tid >= d ? scan[tid - d] : 0u;
+            __syncthreads();
+            scan[tid] += u;
+            __syncthreads();
+        }
+        const std::uint32_t before = scan[tid] - v;
+        __syncthreads();
+        return before;
+    };
+    at[tid] = exclusive(at[tid]);
+    __syncthreads();
+    for (std::uint32_t r0 = tid; r0 < rows; r0 += 4096u) {
+#pragma unroll
+        for (std::uint32_t k = 0; k < 4u; ++k) {
+            const std::uint32_t r = r0 + 1024u * k;
+            if (r >= rows) continue;
+            const int l = row_ptr[r + 1] - row_ptr[r];
+            const std::uint32_t len = l > 0 ? static_cast<std::uint32_t>(l) : 0u;
+            const std::uint32_t slot = slot_of(atomicAdd(&at[bucket_of(len)], 1u), p.sets * kWaves);
+            p.order[slot] = r;
+            p.row_slot[r] = slot;
+            atomicAdd(&load[slot / kSetRows], len);
+        }
+    }
+    __syncthreads();
+    // ranges per set in proportion to its cost, one at least and max_items in all
+    std::uint64_t total = 0u;
+    const std::uint64_t fixed = static_cast<std::uint64_t>(p.parts) * kPartEntries;
+    for (std::uint32_t s = 0; s < p.sets; ++s) total += load[s] + fixed;
+    const std::uint64_t cost = tid < p.sets ? load[tid] + fixed : 0u;
+    std::uint32_t n = 0u;
+    if (tid < p.sets)
+        n = min(static_cast<std::uint32_t>(cost * (p.max_items - p.sets) / total) + 1u, p.parts);
+    const std::uint32_t first = exclusive(n);
+    if (tid < p.sets) {
+        p.splits[tid] = n;
+        p.first[tid] = first;
+        for (std::uint32_t k = 0; k < n; ++k)
+            p.items[first + k] = Item{tid, static_cast<std::uint32_t>(static_cast<std::uint64_t>(p.parts) * k / n),
+                                      static_cast<std::uint32_t>(static_cast<std::uint64_t>(p.parts) * (k + 1u) / n), k};
+    }
+    if (tid == 1023u) scan[0] = first + n;
+    __syncthreads();
+    for (std::uint32_t i = scan[0] + tid; i < p.max_items; i += 1024u) p.items[i] = Item{kNone, 0u, 0u, 0u};
+}
+
+// Lane n of the 16-lane row, to all of it: n is a constant in the unrolled steps.
+template<int kN>
+__device__ __forceinline__ std::uint32_t bcast16(std::uint32_t v) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x150 + kN, 0xf, 0xf, true));
+}
+
+template<int kN>
+__device__ __forceinline__ void step(const char *lane_base, std::uint32_t off, float x, float4 &s) {
+    const float4 g = *reinterpret_cast<const float4 *>(lane_base + bcast16<kN>(off));
+    // The compiler leaves a v_mov_b32_dpp per step where v_fmac_f32 could take the broadcast
+    // itself. s_nop: a DPP operand may not be read within two states of a VALU write.
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(s.x), "+v"(s.y), "+v"(s.z), "+v"(s.w)
+        : "v"(x), "v"(g.x), "v"(g.y), "v"(g.z), "v"(g.w), "n"(kN));
+}
+
+template<int kN>
+__device__ __forceinline__ void step4(const char *lane_base, std::uint32_t off, float x, float4 &s) {
+    step<kN>(lane_base, off, x, s);
+    step<kN + 1>(lane_base, off, x, s);
+    step<kN + 2>(lane_base, off, x, s);
+    step<kN + 3>(lane_base, off, x, s);
+}
+
+// First entry of [b, e) whose column is >= c (the columns ascend), 16 probes a round; the same
+// answer in every range that asks, whatever the order of the columns.
+__device__ __forceinline__ void search(const std::int32_t *col, std::uint32_t c, std::uint32_t (&lo)[kLayers],
+                                       std::uint32_t (&hi)[kLayers], int lane) {
+    const std::uint32_t i16 = static_cast<std::uint32_t>(lane) % 16u;
+    const int shift = (lane / 16) * 16;
+    for (;;) {
+        std::uint32_t left = 0u;
+        std::int32_t v[kLayers];
+#pragma unroll
+        for (int l = 0; l < kLayers; ++l) {
+            const std::uint32_t step = (hi[l] - lo[l] + 16u) / 17u;
+            const std::uint32_t at = lo[l] + (i16 + 1u) * step - 1u;
+            v[l] = step != 0u && at < hi[l] ? col[at] : INT32_MAX;
+        }
+#pragma unroll
+        for (int l = 0; l < kLayers; ++l) {
+            const std::uint32_t step = (hi[l] - lo[l] + 16u) / 17u;
+            const std::uint64_t below = __builtin_amdgcn_ballot_w64(v[l] < static_cast<std::int32_t>(c));
+            const std::uint32_t n = static_cast<std::uint32_t>(__builtin_ctz(~static_cast<std::uint32_t>((below >> shift) & 0xffffu)));
+            lo[l] += n * step;
+            hi[l] = n < 16u ? min(hi[l], lo[l] + step - (step != 0u ? 1u : 0u)) : hi[l];
+            left |= hi[l] - lo[l];
+        }
+        if (__builtin_amdgcn_ballot_w64(left != 0u) == 0ull) return;
+    }
+}
+
+struct Args {
+    const std::int32_t *row_ptr;
+    const std::int32_t *col_idx;
+    const float *values;
+    const float *g;
+    std::int64_t g_ld;
+    std::uint32_t rows, cols;
+    Plan plan;
+};
+
+__global__ __launch_bounds__(kWaves * kWave) void csr_parts_walk(Args a) {
+    __shared__ __attribute__((aligned(16))) char g_part[(kCells + 1) * 256];
+    __shared__ std::uint32_t ends[kSetRows];  // each row's last entry of the range + 1 (not in registers: they are full)
+    const Item item = a.plan.items[blockIdx.x];
+    if (item.set == kNone) return;
+    const int tid = static_cast<int>(threadIdx.x);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lane = tid % kWave;
+    const std::uint32_t i16 = static_cast<std::uint32_t>(lane) % 16u;
+    const int shift = (lane / 16) * 16;
+    if (tid < 16) *reinterpret_cast<float4 *>(g_part + kZeroRow + tid * 16) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+
+    const std::uint32_t *order = a.plan.order + (item.set * kWaves + wave) * (kLayers * 4u) + lane / 16;
+    std::uint32_t cur[kLayers];
+    std::uint32_t *my_ends = ends + wave * (kLayers * 4) + lane / 16;  // read and written by this wave alone
+    {
+        std::uint32_t lo[kLayers], hi[kLayers];
+        auto whole_rows = [&] {
+#pragma unroll
+            for (int l = 0; l < kLayers; ++l) {
+                const std::uint32_t row = order[l * 4];
+                lo[l] = row != kNone ? static_cast<std::uint32_t>(a.row_ptr[row]) : 0u;
+                hi[l] = row != kNone ? max(static_cast<std::uint32_t>(a.row_ptr[row + 1]), lo[l]) : 0u;
+            }
+        };
+        whole_rows();
+        if (item.part1 < a.plan.parts) {
+            search(a.col_idx, item.part1 * kCells, lo, hi, lane);
+#pragma unroll
+            for (int l = 0; l < kLayers; ++l) my_ends[l * 4] = lo[l];
+        } else {
+#pragma unroll
+            for (int l = 0; l < kLayers; ++l) my_ends[l * 4] = hi[l];
+        }
+        whole_rows();
+        if (item.part0 > 0u) search(a.col_idx, item.part0 * kCells, lo, hi, lane);
+#pragma unroll
+        for (int l = 0; l < kLayers; ++l) cur[l] = lo[l];
+    }
+
+    float4 acc[kLayers];
+    std::uint32_t col[kLayers];
+    float val[kLayers];
+    auto load_window = [&](int l) {
+        const std::uint32_t i = cur[l] + i16;
+        col[l] = kNone;
+        val[l] = 0.0f;
+        if (i < my_ends[l * 4]) {
+            col[l] = static_cast<std::uint32_t>(a.col_idx[i]);
+            val[l] = a.values[i];
+        }
+    };
+#pragma unroll
+    for (int l = 0; l < kLayers; ++l) {
+        acc[l] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        load_window(l);
+    }
+
+    const char *lane_base = g_part + i16 * 16u;
+    const std::uint32_t row_bytes = static_cast<std::uint32_t>(a.g_ld) * 4u;
+    const std::uint32_t copy_lane = static_cast<std::uint32_t>(lane / 16) * row_bytes + i16 * 16u;
+    for (std::uint32_t part = item.part0; part < item.part1; ++part) {
+        const std::uint32_t lo = part * kCells;
+        const std::uint32_t span = min(static_cast<std::uint32_t>(kCells), a.cols - lo);
+        __syncthreads();  // every wave is done reading the part before
+#pragma unroll
+        for (int k = 0; k < kCells / 4 / kWaves; ++k) {  // 1 KB, 4 rows, per wave load
+            const std::uint32_t r0 = static_cast<std::uint32_t>(k * kWaves + wave) * 4u;
+            const std::uint32_t left = r0 < span ? min(4u, span - r0) : 0u;
+            const rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float *>(a.g + static_cast<std::int64_t>(lo + r0) * a.g_ld), static_cast<short>(0),
+                left != 0u ? static_cast<int>((left - 1u) * row_bytes + 256u) : 0, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (lds_ptr)(g_part + r0 * 256u), 16, copy_lane, 0, 0, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the copy
+        __syncthreads();
+#pragma unroll
+        for (int l = 0; l < kLayers; ++l) {
+            set_wave_priority(3 - l * 4 / kLayers);  // a wave that is behind issues first (qcsr_spmm_stream)
+            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (;;) {
+                const std::uint32_t rel = col[l] - lo;
+                const std::uint64_t in = __builtin_amdgcn_ballot_w64(rel < span);
+                if (in == 0ull) break;
+                const std::uint32_t cnt = static_cast<std::uint32_t>(__builtin_ctz(~static_cast<std::uint32_t>((in >> shift) & 0xffffu)));
+                const bool mine = i16 < cnt;
+                const std::uint32_t off = mine ? rel * 256u : kZeroRow;
+                const float x = mine ? val[l] : 0.0f;
+                cur[l] += cnt;
+                load_window(l);
+                // the longest prefix of the four groups
+                const std::uint32_t out0 = ~static_cast<std::uint32_t>(in), out1 = ~static_cast<std::uint32_t>(in >> 32);
+                const int n0 = __builtin_ctz(out0 | 0x10000u), n1 = __builtin_ctz((out0 >> 16) | 0x10000u);
+                const int n2 = __builtin_ctz(out1 | 0x10000u), n3 = __builtin_ctz((out1 >> 16) | 0x10000u);
+                const int longest = max(max(n0, n1), max(n2, n3));
+                if (longest == 0) break;  // columns out of order: left to the last kernel
+                step4<0>(lane_base, off, x, s);
+                if (longest > 4) step4<4>(lane_base, off, x, s);
+                if (longest > 8) step4<8>(lane_base, off, x, s);
+                if (longest > 12) step4<12>(lane_base, off, x, s);
+                if (longest < 16) break;
+            }
+            acc[l].x += s.x;
+            acc[l].y += s.y;
+            acc[l].z += s.z;
+            acc[l].w += s.w;
+        }
+    }
+
+    float4 *out = reinterpret_cast<float4 *>(a.plan.partials)
+        + (static_cast<std::uint64_t>(blockIdx.x) * kSetRows + wave * (kLayers * 4u) + lane / 16) * 16u + i16;
+#pragma unroll
+    for (int l = 0; l < kLayers; ++l) {
+        out[l * 64] = acc[l];
+        if (i16 == 0u && cur[l] != my_ends[l * 4]) {
+            const std::uint32_t row = order[l * 4];
+            if (row != kNone) a.plan.broken[row] = 1u;
+        }
+    }
+}
+
+// One wave per row, lane = column: the row's ranges in order, or its entries one by one.
+__global__ __launch_bounds__(256) void csr_parts_reduce(Args a, float *out, std::int64_t out_ld) {
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const std::uint32_t row = blockIdx.x * 4u + threadIdx.x / kWave;
+    if (row >= a.rows) return;
+    float v = 0.0f;
+    if (a.plan.broken[row] == 0u) {
+        const std::uint32_t slot = a.plan.row_slot[row], set = slot / kSetRows;
+        const std::uint32_t n = a.plan.splits[set];
+        const float *p = a.plan.partials + (static_cast<std::uint64_t>(a.plan.first[set]) * kSetRows + slot % kSetRows) * 64u + lane;
+        for (std::uint32_t k = 0; k < n; ++k) v += p[static_cast<std::uint64_t>(k) * kSetRows * 64u];
+    } else {
+        for (std::int32_t i = a.row_ptr[row]; i < a.row_ptr[row + 1]; ++i) {
+            const std::uint32_t c = static_cast<std::uint32_t>(a.col_idx[i]);
+            if (c < a.cols) v = __builtin_fmaf(a.values[i], a.g[static_cast<std::int64_t>(c) * a.g_ld + lane], v);
+        }
+    }
+    out[static_cast<std::int64_t>(row) * out_ld + lane] = v;
+}
+
+std::uint64_t up(std::uint64_t v) { return (v + 255u) / 256u * 256u; }
+
+// Items: two rounds of one workgroup per CU (the second evens out what the cost model misses),
+// one on smaller matrices, and at least one per set.
+std::uint32_t max_items(std::uint32_t sets, std::uint64_t nnz) {
+    return std::max(nnz >= 64'000'000u ? 512u : 256u, sets + sets / 2u);
+}
+
+std::uint64_t layout(void *ws, std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz, Plan *p) {
+    p->sets = (rows + kSetRows - 1u) / kSetRows;
+    p->parts = (cols + kCells - 1u) / kCells;
+    p->max_items = max_items(p->sets, nnz);
+    char *at = static_cast<char *>(ws);
+    std::uint64_t used = 0u;
+    auto take = [&](std::uint64_t bytes) {
+        char *q = at + used;
+        used += up(bytes);
+        return q;
+    };
+    p->order = reinterpret_cast<std::uint32_t *>(take(std::uint64_t{p->sets} * kSetRows * 4u));
+    p->row_slot = reinterpret_cast<std::uint32_t *>(take(std::uint64_t{rows} * 4u));
+    p->broken = reinterpret_cast<std::uint32_t *>(take(std::uint64_t{rows} * 4u));
+    p->splits = reinterpret_cast<std::uint32_t *>(take(std::uint64_t{p->sets} * 4u));
+    p->first = reinterpret_cast<std::uint32_t *>(take(std::uint64_t{p->sets} * 4u));
+    p->items = reinterpret_cast<Item *>(take(std::uint64_t{p->max_items} * sizeof(Item)));
+    p->partials = reinterpret_cast<float *>(take(std::uint64_t{p->max_items} * kSetRows * 256u));
+    return used;
+}
+
+} // namespace
+
+// 64-column blocks of an f32 CSR with enough entries to pay for the plan and the part copies:
+// 4 million, and one per 256 (row, column) pairs (a visit to a layer of four rows in a part
+// costs about 70 instructions a wave, its entries about 7 each four).
+bool csr_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz, std::int64_t n) {
+    return rows > 0u && rows <= kMaxRows && cols > 0u && cols <= static_cast<std::uint32_t>(INT32_MAX) - kCells && n > 0
+        && n % 64 == 0 && n <= 256 && nnz >= 4'000'000u && nnz <= static_cast<std::uint64_t>(INT32_MAX)
+        && nnz * 256u >= static_cast<std::uint64_t>(rows) * cols;
+}
+
+std::uint64_t csr_parts_bytes(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz) {
+    Plan p{};
+    return layout(nullptr, rows, cols, nnz, &p) + 256u;
+}
+
+int launch_csr_parts(const cx_qcsr_matrix &m, const float *g, std::int64_t g_ld, std::int64_t n, float *out,
+                     std::int64_t out_ld, void *workspace, hipStream_t stream) {
+    Args a{};
+    a.row_ptr = m.row_ptr;
+    a.col_idx = m.col_idx;
+    a.values = static_cast<const float *>(m.values);
+    a.g_ld = g_ld;
+    a.rows = m.rows;
+    a.cols = m.cols;
+    void *ws = reinterpret_cast<void *>((reinterpret_cast<std::uintptr_t>(workspace) + 255u) & ~std::uintptr_t{255u});
+    layout(ws, m.rows, m.cols, m.nnz, &a.plan);
+    hipLaunchKernelGGL(csr_parts_plan, dim3(1), dim3(1024), 0, stream, m.row_ptr, m.rows, a.plan);
+    for (std::int64_t c0 = 0; c0 < n; c0 += 64) {
+        a.g = g + c0;
+        hipLaunchKernelGGL(csr_parts_walk, dim3(a.plan.max_items), dim3(kWaves * kWave), 0, stream, a);
+        hipLaunchKernelGGL(csr_parts_reduce, dim3((m.rows + 3u) / 4u), dim3(256), 0, stream, a, out + c0, out_ld);
+    }
+    return check_launch("csr_parts");
+}
+
+} // namespace cx

@@ -426,6 +426,16 @@ extern "C" int cx_qcsr_spmm_bwd_rhs(const cx_qcsr_matrix *transposed, const floa
     if (transposed->bits != 0u || transposed->value_dtype != CELLERATOR_DTYPE_F32)
         return fail(CX_STATUS_INVALID_ARGUMENT,
                     "cx_qcsr_spmm_bwd_rhs: expects the f32 transpose built by cx_qcsr_transpose");
+    // Over LDS parts of grad_out where that pays and the operands are what it reads; every
+    // refusal is the balanced form's.
+    const auto aligned16 = [](const void *p) { return p != nullptr && (reinterpret_cast<std::uintptr_t>(p) & 15u) == 0u; };
+    if (csr_parts_applicable(transposed->rows, transposed->cols, transposed->nnz, out_cols) && aligned16(grad_out)
+        && aligned16(grad_rhs) && aligned16(workspace) && transposed->row_ptr != nullptr && transposed->col_idx != nullptr
+        && transposed->values != nullptr && grad_out_ld >= out_cols && grad_out_ld % 4 == 0 && grad_out_ld <= (1 << 27)
+        && grad_rhs_ld >= out_cols && static_cast<const void *>(grad_rhs) != grad_out
+        && workspace_bytes >= csr_parts_bytes(transposed->rows, transposed->cols, transposed->nnz))
+        return launch_csr_parts(*transposed, grad_out, grad_out_ld, out_cols, grad_rhs, grad_rhs_ld, workspace,
+                                static_cast<hipStream_t>(stream));
     // gene rows of an expression matrix are heavily skewed: the balanced form
     return cx_qcsr_spmm_fwd_balanced(transposed, grad_out, CELLERATOR_DTYPE_F32, grad_out_ld,
                                      out_cols, grad_rhs, grad_rhs_ld, nullptr, workspace,

@@ -143,6 +143,12 @@ bool qcsr_parts_applicable(const QcsrArgs &a, std::uint32_t bits, std::uint32_t 
                            std::int64_t out_cols, bool aligned);
 int launch_qcsr_parts(const QcsrArgs &a, std::uint32_t bits, std::uint32_t policy, std::int64_t out_cols,
                       hipStream_t stream);
+// Y = A . G over LDS parts of G for an unquantized f32 CSR and f32 G (csr_parts.hip): whole
+// 64-column blocks, 16-byte aligned operands, a workspace of csr_parts_bytes.
+bool csr_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz, std::int64_t n);
+std::uint64_t csr_parts_bytes(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz);
+int launch_csr_parts(const cx_qcsr_matrix &m, const float *g, std::int64_t g_ld, std::int64_t n, float *out,
+                     std::int64_t out_ld, void *workspace, hipStream_t stream);
 // grad_values of the backward pass by gene part (fp16 weights, N = 64).
 bool bwd_values_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint32_t rhs_dtype,
                                  std::int64_t out_cols, bool aligned, std::int64_t rhs_ld);
@@ -150,6 +156,16 @@ int launch_bwd_values_parts(const std::int32_t *row_ptr, const std::int32_t *col
                             std::int64_t grad_out_ld, const void *rhs, std::int64_t rhs_ld,
                             float *grad_values, std::uint32_t rows, std::uint32_t cols, bool sorted,
                             hipStream_t stream);
+
+// Issue priority of this wave, 0 .. 3 (p folds to a constant in the unrolled layer loops).
+__device__ __forceinline__ void set_wave_priority(int p) {
+    switch (p) {
+    case 0: __builtin_amdgcn_s_setprio(0); break;
+    case 1: __builtin_amdgcn_s_setprio(1); break;
+    case 2: __builtin_amdgcn_s_setprio(2); break;
+    default: __builtin_amdgcn_s_setprio(3); break;
+    }
+}
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");

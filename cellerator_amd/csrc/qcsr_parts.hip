@@ -29,16 +29,6 @@ namespace {
 constexpr int kPartGenes = 1024;                 // 128 KB of fp16 weight rows per part
 constexpr std::uint32_t kNoRow = 0xffffffffu;
 
-// Issue priority of this wave, 0 .. 3 (p folds to a constant in the unrolled layer loops).
-__device__ __forceinline__ void set_wave_priority(int p) {
-    switch (p) {
-    case 0: __builtin_amdgcn_s_setprio(0); break;
-    case 1: __builtin_amdgcn_s_setprio(1); break;
-    case 2: __builtin_amdgcn_s_setprio(2); break;
-    default: __builtin_amdgcn_s_setprio(3); break;
-    }
-}
-
 using rsrc_t = __amdgpu_buffer_rsrc_t;
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *base, std::uint32_t bytes) {

@@ -463,8 +463,12 @@ int cx_qcsr_spmm_bwd_values(const cx_qcsr_matrix *a, const float *grad_out,
                             int64_t rhs_ld, int64_t out_cols, float *grad_values, void *stream);
 
 /* grad_rhs[cols x out_cols] = A^T . grad_out, with `transposed` the f32 transpose built by
- * cx_qcsr_transpose: cx_qcsr_spmm_fwd_balanced on A^T (workspace sized by
- * cx_qcsr_spmm_balanced_workspace(transposed, out_cols)), every element in a fixed order. Replaces csr_spmm_bwd_rhs_f16_f32 (src/compute/sparse/ops/ops.hh:122-133,
+ * cx_qcsr_transpose (workspace sized by cx_qcsr_spmm_balanced_workspace(transposed, out_cols)),
+ * every element in a fixed order. From 4 million entries on, with out_cols a multiple of 64 up
+ * to 256 and 16-byte aligned operands, grad_out streams through LDS in parts of 512 cells
+ * (columns outside [0, cols) add nothing there); otherwise, and with a workspace that only holds
+ * the balanced form's partial rows, cx_qcsr_spmm_fwd_balanced on A^T. Replaces
+ * csr_spmm_bwd_rhs_f16_f32 (src/compute/sparse/ops/ops.hh:122-133,
  * kernels/base_sparse/csr_spmm_bwd_rhs_kernel_.cuh), which zero-fills grad_rhs and adds
  * with float atomics. */
 int cx_qcsr_spmm_bwd_rhs(const cx_qcsr_matrix *transposed, const float *grad_out,

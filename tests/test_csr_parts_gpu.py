@@ -1,0 +1,75 @@
+"""grad_rhs over LDS parts of grad_out (csr_parts.hip) at the sizes its dispatch takes: ragged
+parts and sets, empty and full rows, several column blocks, rows the part walk cannot finish."""
+from __future__ import annotations
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(rows, cols, mean, seed):
+    import torch
+
+    from cellerator_amd import qcsr_transpose
+    from cellerator_amd.synth import QcsrConfig, generate_qcsr
+    m = generate_qcsr(QcsrConfig("parts", rows, cols, 8, mean, 0.5, zipf_s=1.1, seed=seed))
+    t = qcsr_transpose(m)
+    assert m.nnz >= 4_000_000 and m.nnz * 256 >= rows * cols
+    row = torch.repeat_interleave(torch.arange(cols, device="cuda"), (t.row_ptr[1:] - t.row_ptr[:-1]).long())
+    return m, t, row
+
+
+def _reference(t, row, g, keep=None):
+    import torch
+    a = torch.zeros((t.rows, t.cols), dtype=torch.float64, device="cuda")
+    k = slice(None) if keep is None else keep
+    a.index_put_((row[k], t.col_idx[k].long()), t.values[k].double(), accumulate=True)
+    return a @ g.double(), a.abs() @ g.double().abs()
+
+
+def _check(got, ref, mag):
+    # tests/helpers.py's bound: 1e-4 relative plus 2^-20 of the magnitudes summed
+    assert ((got.double() - ref).abs() <= 1e-4 * ref.abs() + 2.0 ** -20 * mag).all()
+
+
+@pytest.mark.parametrize("rows,cols,mean,n", [(20_000, 700, 260.0, 64), (513 * 12, 2_000, 900.0, 128),
+                                              (40_001, 641, 150.0, 192), (4_100, 6_000, 1_400.0, 64),
+                                              (511, 33_538, 9_000.0, 256)])
+def test_grad_rhs_parts(rows, cols, mean, n):
+    import torch
+
+    from cellerator_amd import qcsr_spmm_bwd_rhs
+    m, t, row = _matrix(rows, cols, mean, seed=rows)
+    wide = torch.randn((rows, n + 4), device="cuda")
+    for g in (wide[:, :n].contiguous(), wide[:, :n]):
+        got = qcsr_spmm_bwd_rhs(t, g)
+        _check(got, *_reference(t, row, g))
+        assert torch.equal(got, qcsr_spmm_bwd_rhs(t, g))
+
+
+def test_grad_rhs_parts_disorder_and_infinities():
+    """Columns shuffled in a few rows and pointing outside the matrix in others (those rows are
+    summed entry by entry; the stray entries add nothing), and infinite rows of grad_out, which
+    may reach the rows that hold them only."""
+    import torch
+
+    from cellerator_amd import qcsr_spmm_bwd_rhs
+    m, t, row = _matrix(20_000, 700, 260.0, seed=9)
+    g = torch.randn((20_000, 64), device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    for r in (0, 5, 300, 699):
+        b, e = int(t.row_ptr[r]), int(t.row_ptr[r + 1])
+        p = torch.randperm(e - b, device="cuda", generator=gen)
+        t.col_idx[b:e], t.values[b:e] = t.col_idx[b:e][p], t.values[b:e][p]
+    keep = torch.ones(t.nnz, dtype=torch.bool, device="cuda")
+    for r, c in ((5, 20_000), (17, -1), (400, 2**31 - 1), (650, 20_480)):
+        at = int(t.row_ptr[r]) + (int(t.row_ptr[r + 1]) - int(t.row_ptr[r])) // 2
+        t.col_idx[at] = c
+        keep[at] = False
+    keep = keep.nonzero().flatten()
+    _check(qcsr_spmm_bwd_rhs(t, g), *_reference(t, row, g, keep))
+    g[100] = float("inf")
+    held = torch.zeros(700, dtype=torch.bool, device="cuda")
+    held[row[keep][(t.col_idx[keep] == 100) & (t.values[keep] != 0)]] = True
+    got = qcsr_spmm_bwd_rhs(t, g)
+    assert torch.equal(torch.isfinite(got).all(dim=1), ~held)
