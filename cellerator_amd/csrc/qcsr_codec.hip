@@ -12,10 +12,19 @@
 // block's first entry. Per-gene affine, interleaved (scale, offset) pairs and column scale
 // with row offset metadata; a null scale reads 1, a null offset 0.
 //
-// Layout of the work: one wave per row, lanes over the row's packed bytes (quantize: each lane
-// assembles a whole byte, so there is no read-modify-write of shared bytes and adjacent lanes
-// store adjacent bytes) or over its entries (dequantize: adjacent lanes store adjacent fp32
-// values); four rows per workgroup, rows of the block strided over the grid.
+// Layout of the work: one wave per row; a lane takes 4 consecutive entries at a time (8 of one
+// bit), so its columns and values move 16 bytes at once and its codes are whole bytes: no
+// read-modify-write of shared bytes, and rows need no alignment. Two such groups are in flight
+// per wave.
+//
+// The per-gene metadata is the cost: gathered per entry through the texture path (two arrays, a
+// lane's address each) it took 2 of the 3.5 cycles per entry and CU. On larger blocks one
+// workgroup of 16 waves per CU keeps 20,000 genes' (scale, offset) pairs (40,000 scales under row
+// offsets) in LDS. Past that many genes the rows are walked twice, with the next genes' metadata:
+// a lane's entries belong to the phase of their furthest gene (ascending columns: whole
+// stretches of the row), which costs a second read of the columns and no gathers up to 40,000
+// genes; the rest are gathered in the second walk. 75M 4-bit entries of 20,000 genes decode in 193 us
+// and encode in 209 (3.3 and 3.0 TB/s of columns, codes and values), 455 and 610 gathered.
 #include "qcsr_common.hpp"
 
 namespace cx {
@@ -37,15 +46,6 @@ struct CodecArgs {
     std::int64_t nnz_begin;  // values are indexed from this entry
 };
 
-__device__ __forceinline__ float2 entry_meta(const CodecArgs &a, std::int32_t row, std::int32_t col) {
-    if (a.policy == CX_DECODE_PER_GENE_AFFINE_PAIRS) return reinterpret_cast<const float2 *>(a.scales)[col];
-    const float s = a.scales != nullptr ? a.scales[col] : 1.0f;
-    float o;
-    if (a.policy == CX_DECODE_COLUMN_SCALE_ROW_OFFSET) o = a.row_offsets != nullptr ? a.row_offsets[row] : 0.0f;
-    else o = a.offsets != nullptr ? a.offsets[col] : 0.0f;
-    return make_float2(s, o);
-}
-
 template<int kBits>
 __device__ __forceinline__ std::uint32_t encode(float value, float2 md) {
     if (md.x == 0.0f) return 0u;
@@ -55,53 +55,170 @@ __device__ __forceinline__ std::uint32_t encode(float value, float2 md) {
     return static_cast<std::uint32_t>(r > (1 << kBits) - 1 ? (1 << kBits) - 1 : r);
 }
 
-template<int kBits>
-__global__ __launch_bounds__(kCodecWaves * kWave) void quantize_rows_kernel(CodecArgs a, const float *values,
-                                                                            std::uint8_t *packed) {
-    constexpr int kPerByte = 8 / kBits;
-    const int lane = static_cast<int>(threadIdx.x) % kWave;
-    for (std::int64_t row = a.row_begin + static_cast<std::int64_t>(blockIdx.x) * kCodecWaves + threadIdx.x / kWave;
-         row < a.row_end; row += static_cast<std::int64_t>(gridDim.x) * kCodecWaves) {
-        const std::int64_t begin = a.row_ptr[row], end = a.row_ptr[row + 1];
-        const std::int64_t out0 = a.packed_row_ptr[row];
-        const std::int64_t bytes = (end - begin + kPerByte - 1) / kPerByte;
-        for (std::int64_t b = lane; b < bytes; b += kWave) {
-            std::uint32_t byte = 0u;
-#pragma unroll
-            for (int k = 0; k < kPerByte; ++k) {
-                const std::int64_t i = begin + b * kPerByte + k;
-                if (i < end) {
-                    // a column outside [0, cols) (a broken structure) encodes as code 0
-                    const std::int32_t col = a.col_idx[i];
-                    if (static_cast<std::uint32_t>(col) < a.cols)
-                        byte |= encode<kBits>(values[i - a.nnz_begin], entry_meta(a, static_cast<std::int32_t>(row), col))
-                            << (k * kBits);
-                }
-            }
-            packed[out0 + b] = static_cast<std::uint8_t>(byte);
+// Metadata of the entries a lane holds: genes [first, first + staged) from LDS, the rest
+// gathered; a column outside [0, cols) (a broken structure) reads (0, 0): it encodes as code 0, decodes as 0.
+template<bool kRowOffset>
+struct Meta {
+    const char *lds;
+    std::uint32_t first, staged;
+    float row_offset;
+
+    __device__ __forceinline__ float2 of(const CodecArgs &a, std::uint32_t col) const {
+        float2 md = make_float2(0.0f, 0.0f);
+        if (col - first < staged) {
+            if constexpr (kRowOffset) md.x = reinterpret_cast<const float *>(lds)[col - first];
+            else md = reinterpret_cast<const float2 *>(lds)[col - first];
+        } else if (col < a.cols) {
+            if constexpr (kRowOffset) md.x = a.scales != nullptr ? a.scales[col] : 1.0f;
+            else if (a.policy == CX_DECODE_PER_GENE_AFFINE_PAIRS) md = reinterpret_cast<const float2 *>(a.scales)[col];
+            else md = make_float2(a.scales != nullptr ? a.scales[col] : 1.0f, a.offsets != nullptr ? a.offsets[col] : 0.0f);
+        }
+        if constexpr (kRowOffset) md.y = col < a.cols ? row_offset : 0.0f;
+        return md;
+    }
+};
+
+// Entries a lane takes at a time: 16 bytes of columns and values, and whole code bytes where it
+// writes them.
+template<int kBits, bool kEncode>
+constexpr int kLaneEntries = kBits == 1 && kEncode ? 8 : 4;
+
+constexpr int kGroups = 2;
+
+// kWhole: a wave per row (row_lanes_arg is then kWave).
+template<int kBits, bool kEncode, bool kRowOffset, bool kWhole>
+__global__ __launch_bounds__(16 * kWave) void codec_rows_kernel(CodecArgs a, const float *values_in, const std::uint8_t *packed_in,
+                                                                float *values_out, std::uint8_t *packed_out,
+                                                                std::uint32_t row_lanes_arg, std::uint32_t stage,
+                                                                std::uint32_t phases) {
+    constexpr int kE = kLaneEntries<kBits, kEncode>;
+    constexpr int kB = (kE * kBits + 7) / 8;  // code bytes of a lane's entries
+    constexpr std::uint32_t kMask = (1u << kBits) - 1u;
+    extern __shared__ __attribute__((aligned(16))) char meta_lds[];
+    __shared__ std::uint32_t next_row;
+    const std::uint32_t row_lanes = kWhole ? static_cast<std::uint32_t>(kWave) : row_lanes_arg;
+    const std::uint32_t lane = threadIdx.x % row_lanes, wg_rows = blockDim.x / row_lanes;
+    const std::uint32_t nnz_begin = static_cast<std::uint32_t>(a.nnz_begin);
+    for (std::uint32_t phase = 0; phase < phases; ++phase) {
+    if (phase != 0u) __syncthreads();  // every row of the phase before is done
+    if (threadIdx.x == 0u) next_row = wg_rows;
+    const std::uint32_t first = phase * stage, staged = min(stage, a.cols - first);
+    if (stage != 0u) {
+        for (std::uint32_t g = threadIdx.x; g < staged; g += blockDim.x) {
+            const float scale = a.scales != nullptr && a.policy != CX_DECODE_PER_GENE_AFFINE_PAIRS ? a.scales[first + g] : 1.0f;
+            if constexpr (kRowOffset) reinterpret_cast<float *>(meta_lds)[g] = scale;
+            else if (a.policy == CX_DECODE_PER_GENE_AFFINE_PAIRS)
+                reinterpret_cast<float2 *>(meta_lds)[g] = reinterpret_cast<const float2 *>(a.scales)[first + g];
+            else
+                reinterpret_cast<float2 *>(meta_lds)[g] = make_float2(scale, a.offsets != nullptr ? a.offsets[first + g] : 0.0f);
         }
     }
-}
-
-template<int kBits>
-__global__ __launch_bounds__(kCodecWaves * kWave) void dequantize_rows_kernel(CodecArgs a, const std::uint8_t *packed,
-                                                                              float *values) {
-    constexpr int kPerByte = 8 / kBits;
-    constexpr std::uint32_t kMask = (1u << kBits) - 1u;
-    const int lane = static_cast<int>(threadIdx.x) % kWave;
-    for (std::int64_t row = a.row_begin + static_cast<std::int64_t>(blockIdx.x) * kCodecWaves + threadIdx.x / kWave;
-         row < a.row_end; row += static_cast<std::int64_t>(gridDim.x) * kCodecWaves) {
-        const std::int64_t begin = a.row_ptr[row], end = a.row_ptr[row + 1];
-        const std::uint8_t *in = packed + a.packed_row_ptr[row];
-        for (std::int64_t i = begin + lane; i < end; i += kWave) {
-            const std::int64_t local = i - begin;
-            const std::uint32_t code = (static_cast<std::uint32_t>(in[local / kPerByte]) >> ((local % kPerByte) * kBits)) & kMask;
-            const std::int32_t col = a.col_idx[i];
-            // a column outside [0, cols) (a broken structure) decodes as 0
-            const float2 md = static_cast<std::uint32_t>(col) < a.cols
-                ? entry_meta(a, static_cast<std::int32_t>(row), col) : make_float2(0.0f, 0.0f);
-            values[i - a.nnz_begin] = __builtin_fmaf(static_cast<float>(code), md.x, md.y);
+    __syncthreads();
+    // The workgroup's rows (every gridDim-th) go to its waves first come, first served: dealt
+    // ahead, the wave with the longest 12 of 50k log-normal rows ended well after the mean
+    // (encoding 75M entries 236 -> 210 us). Several rows a wave are dealt.
+    std::uint32_t at = threadIdx.x / row_lanes;
+    for (;;) {
+        const std::int64_t row = a.row_begin + static_cast<std::int64_t>(at) * gridDim.x + blockIdx.x;
+        if (row >= a.row_end) break;
+        if constexpr (kWhole) {
+            if (lane == 0u) at = atomicAdd(&next_row, 1u);
+            at = static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
+        } else {
+            at += wg_rows;
         }
+        // entry offsets are below 2^31, so 32-bit sums of them and a step do not wrap
+        const std::uint32_t begin = static_cast<std::uint32_t>(a.row_ptr[row]), end = static_cast<std::uint32_t>(a.row_ptr[row + 1]);
+        const std::uint32_t bytes0 = static_cast<std::uint32_t>(a.packed_row_ptr[row]);
+        Meta<kRowOffset> meta{meta_lds, first, staged, 0.0f};
+        if constexpr (kRowOffset) meta.row_offset = a.row_offsets != nullptr ? a.row_offsets[row] : 0.0f;
+
+        struct Held {
+            std::int32_t col[kE];
+            float v[kE];
+            std::uint32_t codes;
+            bool mine;  // holds entries, and its furthest gene belongs to this phase
+        };
+        // entries [i, i + kE) of the row, whole vectors where they all lie in it
+        auto load_cols = [&](Held &h, std::uint32_t i) {
+            if (i + kE <= end) {
+                __builtin_memcpy(h.col, a.col_idx + i, sizeof(h.col));
+            } else {
+#pragma unroll
+                for (int k = 0; k < kE; ++k) h.col[k] = i + k < end ? a.col_idx[i + k] : -1;
+            }
+            h.mine = i < end;
+            if (phases > 1u) {
+                std::uint32_t furthest = 0u;
+#pragma unroll
+                for (int k = 0; k < kE; ++k)
+                    if (static_cast<std::uint32_t>(h.col[k]) < a.cols) furthest = max(furthest, static_cast<std::uint32_t>(h.col[k]));
+                h.mine = h.mine && furthest >= first && (furthest < first + stage || phase + 1u == phases);
+            }
+        };
+        auto load = [&](Held &h, std::uint32_t i) {
+            if (!h.mine) return;
+            if (i + kE <= end) {
+                if constexpr (kEncode) __builtin_memcpy(h.v, values_in + (i - nnz_begin), sizeof(h.v));
+                else {
+                    h.codes = 0u;
+                    __builtin_memcpy(&h.codes, packed_in + bytes0 + (i - begin) * kBits / 8, kB);
+                    if constexpr (kE * kBits < 8) h.codes >>= (i - begin) * kBits % 8;
+                }
+            } else {
+                h.codes = 0u;
+#pragma unroll
+                for (int k = 0; k < kE; ++k) {
+                    if (i + k >= end) continue;
+                    if constexpr (kEncode) h.v[k] = values_in[i + k - nnz_begin];
+                    else
+                        h.codes |= (packed_in[bytes0 + (i + k - begin) * kBits / 8] >> ((i + k - begin) * kBits % 8) & kMask) << (k * kBits);
+                }
+            }
+        };
+        auto finish = [&](const Held &h, std::uint32_t i) {
+            if (!h.mine) return;
+            if constexpr (kEncode) {
+                std::uint32_t codes = 0u;
+#pragma unroll
+                for (int k = 0; k < kE; ++k)
+                    if (h.col[k] >= 0 && static_cast<std::uint32_t>(h.col[k]) < a.cols)
+                        codes |= encode<kBits>(h.v[k], meta.of(a, static_cast<std::uint32_t>(h.col[k]))) << (k * kBits);
+                std::uint8_t *out = packed_out + bytes0 + (i - begin) * kBits / 8;
+                if (i + kE <= end) {
+                    __builtin_memcpy(out, &codes, kB);
+                } else {
+                    const std::uint32_t n = ((end - i) * kBits + 7u) / 8u;
+                    for (std::uint32_t b = 0; b < n; ++b) out[b] = static_cast<std::uint8_t>(codes >> (8 * b));
+                }
+            } else {
+                float v[kE];
+#pragma unroll
+                for (int k = 0; k < kE; ++k) {
+                    const float2 md = meta.of(a, static_cast<std::uint32_t>(h.col[k]));
+                    v[k] = __builtin_fmaf(static_cast<float>((h.codes >> (k * kBits)) & kMask), md.x, md.y);
+                }
+                float *out = values_out + (i - nnz_begin);
+                if (i + kE <= end) {
+                    __builtin_memcpy(out, v, sizeof(v));
+                } else {
+#pragma unroll
+                    for (int k = 0; k < kE; ++k)
+                        if (i + k < end) out[k] = v[k];
+                }
+            }
+        };
+        const std::uint32_t step = row_lanes * kE;
+        for (std::uint32_t i = begin + lane * kE; i < end; i += kGroups * step) {
+            Held h[kGroups];  // all in flight before the first is decoded
+#pragma unroll
+            for (int q = 0; q < kGroups; ++q) load_cols(h[q], i + q * step);
+#pragma unroll
+            for (int q = 0; q < kGroups; ++q) load(h[q], i + q * step);
+#pragma unroll
+            for (int q = 0; q < kGroups; ++q) finish(h[q], i + q * step);
+        }
+    }
     }
 }
 
@@ -141,9 +258,64 @@ int prepare(const cx_qcsr_matrix *m, const cx_qcsr_block *block, CodecArgs *a, c
     return CX_STATUS_SUCCESS;
 }
 
-unsigned codec_grid(const CodecArgs &a) {
+// Bytes of metadata a workgroup keeps in LDS, and the entries from which it does (3 million on
+// 33,538 genes: 39 us gathered, 38 staged; 4.5 million on 20,000: 61 and 29).
+constexpr std::uint32_t kStageBytes = 160'000u;
+constexpr std::int64_t kStageEntries = 4'000'000;
+
+// Lanes per row: a wave's; where there are rows enough to fill the chip anyway, as many as take
+// a row of the mean length in one step of two groups, so a wave has several rows in flight
+// (100k rows of 200 entries).
+template<int kBits, bool kEncode>
+std::uint32_t codec_row_lanes(std::int64_t entries, std::int64_t rows) {
+    std::uint32_t l = kWave;
+    while (l > 8u && rows >= 16384 && static_cast<std::int64_t>(l) * kLaneEntries<kBits, kEncode> * (kGroups / 2) * rows >= entries) l /= 2u;
+    return l;
+}
+
+template<int kBits, bool kEncode, bool kRowOffset>
+void launch_codec(const CodecArgs &a, std::int64_t entries, const float *vin, const std::uint8_t *pin, float *vout,
+                  std::uint8_t *pout, hipStream_t s) {
     const std::int64_t rows = static_cast<std::int64_t>(a.row_end) - a.row_begin;
-    return static_cast<unsigned>(std::min<std::int64_t>((rows + kCodecWaves - 1) / kCodecWaves, 1 << 20));
+    const std::uint32_t lanes = codec_row_lanes<kBits, kEncode>(entries, rows);
+    constexpr std::uint32_t kPer = kRowOffset ? 4u : 8u;
+    const std::uint32_t fits = std::min(a.cols, kStageBytes / kPer);
+    const bool staged = fits != 0u && entries >= 1'000'000 && entries * kStageBytes >= kStageEntries * fits * kPer;
+    const std::uint32_t threads = (staged ? 16u : kCodecWaves) * kWave;
+    const std::int64_t groups = (rows * lanes + threads - 1) / threads;
+    const std::uint32_t stage = staged ? fits : 0u;
+    const std::uint32_t phases = staged && a.cols > stage ? 2u : 1u;
+    const std::int64_t most = staged ? (2u * stage * kPer <= kStageBytes ? 512 : 256) : 1 << 20;
+    const dim3 grid(static_cast<unsigned>(std::min(groups, most))), block(threads);
+    if (lanes == static_cast<std::uint32_t>(kWave))
+        hipLaunchKernelGGL((codec_rows_kernel<kBits, kEncode, kRowOffset, true>), grid, block, stage * kPer, s, a, vin, pin, vout,
+                           pout, lanes, stage, phases);
+    else
+        hipLaunchKernelGGL((codec_rows_kernel<kBits, kEncode, kRowOffset, false>), grid, block, stage * kPer, s, a, vin, pin, vout,
+                           pout, lanes, stage, phases);
+}
+
+template<bool kEncode>
+void launch_codec_bits(const CodecArgs &a, std::uint32_t bits, std::int64_t entries, const float *vin,
+                       const std::uint8_t *pin, float *vout, std::uint8_t *pout, hipStream_t s) {
+    const bool row_offset = a.policy == CX_DECODE_COLUMN_SCALE_ROW_OFFSET;
+#define CX_CODEC(B)                                                                                  \
+    do {                                                                                             \
+        if (row_offset) launch_codec<B, kEncode, true>(a, entries, vin, pin, vout, pout, s);         \
+        else launch_codec<B, kEncode, false>(a, entries, vin, pin, vout, pout, s);                   \
+    } while (0)
+    switch (bits) {
+    case 1: CX_CODEC(1); break;
+    case 2: CX_CODEC(2); break;
+    case 4: CX_CODEC(4); break;
+    default: CX_CODEC(8); break;
+    }
+#undef CX_CODEC
+}
+
+// Entries of the call: the block's, or the matrix's.
+std::int64_t entry_count(const cx_qcsr_matrix *m, const cx_qcsr_block *block) {
+    return block != nullptr ? static_cast<std::int64_t>(block->nnz_end) - block->nnz_begin : static_cast<std::int64_t>(m->nnz);
 }
 
 } // namespace
@@ -190,14 +362,8 @@ extern "C" int cx_qcsr_quantize_block(const cx_qcsr_matrix *m, const cx_qcsr_blo
     if (a.row_end == a.row_begin) return CX_STATUS_SUCCESS;
     if (packed_out == nullptr || (m->nnz != 0u && values_by_nnz_block == nullptr))
         return fail(CX_STATUS_INVALID_ARGUMENT, "cx_qcsr_quantize_block: null values or packed output");
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid(codec_grid(a)), threads(kCodecWaves * kWave);
-    switch (m->bits) {
-    case 1: hipLaunchKernelGGL(quantize_rows_kernel<1>, grid, threads, 0, s, a, values_by_nnz_block, packed_out); break;
-    case 2: hipLaunchKernelGGL(quantize_rows_kernel<2>, grid, threads, 0, s, a, values_by_nnz_block, packed_out); break;
-    case 4: hipLaunchKernelGGL(quantize_rows_kernel<4>, grid, threads, 0, s, a, values_by_nnz_block, packed_out); break;
-    default: hipLaunchKernelGGL(quantize_rows_kernel<8>, grid, threads, 0, s, a, values_by_nnz_block, packed_out); break;
-    }
+    launch_codec_bits<true>(a, m->bits, entry_count(m, block), values_by_nnz_block, nullptr, nullptr, packed_out,
+                            static_cast<hipStream_t>(stream));
     return check_launch("cx_qcsr_quantize_block");
 }
 
@@ -211,14 +377,7 @@ extern "C" int cx_qcsr_dequantize_block(const cx_qcsr_matrix *m, const cx_qcsr_b
     if (a.row_end == a.row_begin) return CX_STATUS_SUCCESS;
     if ((m->nnz != 0u && (values_by_nnz_block == nullptr || m->packed_values == nullptr)))
         return fail(CX_STATUS_INVALID_ARGUMENT, "cx_qcsr_dequantize_block: null values or codes");
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid(codec_grid(a)), threads(kCodecWaves * kWave);
-    const std::uint8_t *p = m->packed_values;
-    switch (m->bits) {
-    case 1: hipLaunchKernelGGL(dequantize_rows_kernel<1>, grid, threads, 0, s, a, p, values_by_nnz_block); break;
-    case 2: hipLaunchKernelGGL(dequantize_rows_kernel<2>, grid, threads, 0, s, a, p, values_by_nnz_block); break;
-    case 4: hipLaunchKernelGGL(dequantize_rows_kernel<4>, grid, threads, 0, s, a, p, values_by_nnz_block); break;
-    default: hipLaunchKernelGGL(dequantize_rows_kernel<8>, grid, threads, 0, s, a, p, values_by_nnz_block); break;
-    }
+    launch_codec_bits<false>(a, m->bits, entry_count(m, block), nullptr, m->packed_values, values_by_nnz_block, nullptr,
+                             static_cast<hipStream_t>(stream));
     return check_launch("cx_qcsr_dequantize_block");
 }

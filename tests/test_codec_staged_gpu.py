@@ -1,0 +1,45 @@
+"""The codec with its metadata staged in LDS (blocks of 4 million entries and more), against the
+same passes over small blocks, which tests/test_codec_gpu.py pins to the host codec."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("policy,cols", [(1, 45_000), (2, 45_000), (3, 45_000), (1, 4_999)])
+def test_staged_codec_equals_small_blocks(bits, policy, cols):
+    """Genes on both sides of the staged range (20,000 pairs, 40,000 scales), rows of every
+    length modulo a lane's entries, entries outside [0, cols)."""
+    import torch
+
+    from cellerator_amd import QcsrMatrix, qcsr_pack_gene_affine
+    from cellerator_amd import _native as N
+    from cellerator_amd.codec import dequantize, get_block, quantize
+    from cellerator_amd.synth import QcsrConfig, generate_qcsr
+    m = generate_qcsr(QcsrConfig("codec", 6_001, cols, bits, 900.0, 0.5, zipf_s=0.4, seed=40 + bits))
+    assert m.nnz >= 4_000_000
+    m.col_idx[torch.tensor([3, 1_000, m.nnz - 1], device="cuda")] = torch.tensor([-1, cols, 2**31 - 1], dtype=torch.int32,
+                                                                               device="cuda")
+    if policy == 2:
+        m = QcsrMatrix(m.rows, cols, bits, m.row_ptr, m.col_idx, packed_row_ptr=m.packed_row_ptr,
+                       packed_values=m.packed_values, column_scales=m.column_scales,
+                       row_offsets=torch.rand(m.rows, device="cuda"), decode_policy=N.DECODE_COLUMN_SCALE_ROW_OFFSET)
+    if policy == 3:
+        m = qcsr_pack_gene_affine(m)
+    values = torch.rand(m.nnz, device="cuda") * 3.0 + 0.2
+    whole, whole_packed = dequantize(m), torch.zeros_like(m.packed_values)
+    quantize(m, values, packed_out=whole_packed)
+    out, packed = torch.full_like(whole, float("nan")), torch.zeros_like(m.packed_values)
+    rp, prp = m.row_ptr.cpu().numpy(), m.packed_row_ptr.cpu().numpy()
+    brp = np.array([0, 1_000, 2_500, m.rows], np.int32)
+    for k in range(3):
+        b = get_block(brp, rp, prp, k)
+        assert b.nnz_end - b.nnz_begin < 4_000_000
+        dequantize(m, out[b.nnz_begin:], block=b)
+        quantize(m, values[b.nnz_begin:].contiguous(), packed_out=packed, block=b)
+    assert torch.equal(whole.view(torch.int32), out.view(torch.int32))
+    assert torch.equal(whole_packed, packed)
+    assert float(whole[3]) == 0.0 and float(whole[m.nnz - 1]) == 0.0
