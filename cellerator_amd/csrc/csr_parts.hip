@@ -221,7 +221,12 @@ struct Args {
 __global__ __launch_bounds__(kWaves * kWave) void csr_parts_walk(Args a) {
     __shared__ __attribute__((aligned(16))) char g_part[(kCells + 1) * 256];
     __shared__ std::uint32_t ends[kSetRows];  // each row's last entry of the range + 1 (not in registers: they are full)
-    const Item item = a.plan.items[blockIdx.x];
+    Item item = a.plan.items[blockIdx.x];
+    // into scalar registers: the load is a vector one, and a part index in vector registers puts the
+    // copy's descriptors in loops
+    item.set = __builtin_amdgcn_readfirstlane(item.set);
+    item.part0 = __builtin_amdgcn_readfirstlane(item.part0);
+    item.part1 = __builtin_amdgcn_readfirstlane(item.part1);
     if (item.set == kNone) return;
     const int tid = static_cast<int>(threadIdx.x);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);

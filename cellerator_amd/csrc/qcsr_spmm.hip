@@ -165,7 +165,7 @@ constexpr std::uint32_t kNoEntry = 0x7fff8000u;
 // read at 32-bit offsets through a buffer descriptor over exactly [cols x N], so an entry whose
 // column lies outside [0, cols), or past the chunk's end, reads zeros and adds nothing.
 template<int kBits, int kPolicy, ValueMode kMode, typename RhsT, int kN>
-__global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int log_split) {
+__global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int log_split, std::uint32_t rhs_bytes) {
     using S = WaveShape<RhsT, kN>;
     constexpr int kCpl = S::kCpl, kLpe = S::kLpe, kEps = S::kEps;
     constexpr int kBatch = 4;  // steps whose gathers are in flight together
@@ -179,9 +179,10 @@ __global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int lo
     const int j = lane % kLpe;
     uint2 *stage = stage_all[wave];
     const std::uint32_t row_bytes = static_cast<std::uint32_t>(a.rhs_ld) * sizeof(RhsT);
-    const auto rw = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<void *>(a.rhs), static_cast<short>(0),
-        a.cols != 0u ? static_cast<int>((a.cols - 1u) * row_bytes + kN * sizeof(RhsT)) : 0, 0x00020000);
+    // (the byte count comes from the host: computed here it ended in vector registers, and every
+    // gather in a loop that makes the descriptor uniform)
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.rhs), static_cast<short>(0),
+                                                      static_cast<int>(rhs_bytes), 0x00020000);
     float acc[kCpl];
 #pragma unroll
     for (int k = 0; k < kCpl; ++k) acc[k] = 0.0f;
@@ -292,7 +293,9 @@ void launch_split(const QcsrArgs &a, int log_split, hipStream_t stream) {
     const int waves = log_split <= 2 ? 4 : 1 << log_split;
     const std::uint32_t rows_per_block = static_cast<std::uint32_t>(waves >> log_split);
     hipLaunchKernelGGL((qcsr_spmm_split<kBits, kPolicy, kMode, RhsT, kN>),
-                       dim3((a.rows + rows_per_block - 1u) / rows_per_block), dim3(waves * kWave), 0, stream, a, log_split);
+                       dim3((a.rows + rows_per_block - 1u) / rows_per_block), dim3(waves * kWave), 0, stream, a, log_split,
+                       a.cols != 0u ? static_cast<std::uint32_t>(((a.cols - 1u) * static_cast<std::uint64_t>(a.rhs_ld) + kN) * sizeof(RhsT))
+                                    : 0u);
 }
 
 // ---- load-balanced form: equal nnz chunks, one wave per chunk ----------------------------
