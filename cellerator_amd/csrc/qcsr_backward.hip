@@ -99,6 +99,97 @@ __global__ __launch_bounds__(kWave *kWavesPerBlock) void qcsr_bwd_values_rowwave
     }
 }
 
+// The row-wave form with 1 to 16 waves per row (every entry is its own result, so a row's 64-entry
+// chunks go to its waves without more ado) and kLpe = 8 or 16 lanes per entry: four gathers in
+// flight, through a descriptor that reads zeros for columns outside [0, cols), and one
+// reduce-scatter per 8 steps, after which every lane holds the result of one entry of the
+// chunk. Bound by the texture path like qcsr_spmm_split. 30,000 x 33,538, 45M entries, N = 128:
+// 746 us, 1,885 with the row-wave form (one gather in flight and a shuffle butterfly per step).
+template<typename RhsT, int kN>
+__global__ __launch_bounds__(16 * kWave) void qcsr_bwd_values_split(BwdValuesArgs a, int log_split, std::uint32_t cols,
+                                                                    std::uint32_t rhs_bytes) {
+    constexpr int kCpl = 16 / static_cast<int>(sizeof(RhsT));
+    constexpr int kLpe = kN / kCpl, kEps = kWave / kLpe, kSteps = kWave / kEps;
+    static_assert(kLpe == 8 || kLpe == 16, "one or two half rows of lanes per entry");
+    __shared__ std::uint32_t stage_all[16][kWave];
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const std::uint32_t row = blockIdx.x * ((blockDim.x / kWave) >> log_split) + (wave >> log_split);
+    if (row >= a.rows) return;
+    const int g = lane / kLpe, j = lane % kLpe;
+    std::uint32_t *stage = stage_all[wave];
+    const std::uint32_t row_bytes = static_cast<std::uint32_t>(a.rhs_ld) * sizeof(RhsT);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.rhs), static_cast<short>(0),
+                                                      static_cast<int>(rhs_bytes), 0x00020000);
+    float go[kCpl];
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(a.grad_out + static_cast<std::int64_t>(row) * a.grad_out_ld + j * kCpl);
+#pragma unroll
+        for (int k = 0; k < kCpl / 4; ++k) {
+            const float4 v = src[k];
+            go[4 * k] = v.x; go[4 * k + 1] = v.y; go[4 * k + 2] = v.z; go[4 * k + 3] = v.w;
+        }
+    }
+    const std::uint32_t end = static_cast<std::uint32_t>(a.row_ptr[row + 1]);
+    const std::uint32_t step = static_cast<std::uint32_t>(kWave) << log_split;
+    std::uint32_t c0 = static_cast<std::uint32_t>(a.row_ptr[row]) + (wave & ((1 << log_split) - 1)) * kWave;
+    auto load_col = [&](std::uint32_t c) { return c + lane < end ? static_cast<std::uint32_t>(a.col_idx[c + lane]) : 0xffffffffu; };
+    std::uint32_t col = load_col(c0);
+    for (; c0 < end; c0 += step) {
+        stage[lane] = col < cols ? col * row_bytes : kNoEntry;
+        wave_sync();
+        col = load_col(c0 + step);
+        float d[kSteps];
+#pragma unroll
+        for (int s0 = 0; s0 < kSteps; s0 += 4) {
+            uint4 w[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, static_cast<int>(stage[(s0 + q) * kEps + g] + j * 16u), 0, 0);
+                w[q] = make_uint4(v[0], v[1], v[2], v[3]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const unsigned words[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
+                float dot = 0.0f;
+                if constexpr (sizeof(RhsT) == 2) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        dot = __builtin_fmaf(go[2 * k], h2f(static_cast<std::uint16_t>(words[k] & 0xffffu)), dot);
+                        dot = __builtin_fmaf(go[2 * k + 1], h2f(static_cast<std::uint16_t>(words[k] >> 16)), dot);
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) dot = __builtin_fmaf(go[k], __uint_as_float(words[k]), dot);
+                }
+                if constexpr (kLpe == 16)  // the half row 8 lanes away
+                    dot += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(dot), 0x128, 0xf, 0xf, true));
+                d[s0 + q] = dot;
+            }
+        }
+        // lane (g, j) holds step j's entry of group g
+        float v = group_scatter8(d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7], j % 8);
+        if constexpr (kLpe == 16) {
+            const float u = group_scatter8(d[8], d[9], d[10], d[11], d[12], d[13], d[14], d[15], j % 8);
+            v = j < 8 ? v : u;
+        }
+        const std::uint32_t e = static_cast<std::uint32_t>(j * kEps + g);
+        if (stage[e] == kNoEntry) v = 0.0f;
+        if (c0 + e < end) a.grad_values[c0 + e] = v;
+        wave_sync();
+    }
+}
+
+template<typename RhsT, int kN>
+void launch_bwd_split(const BwdValuesArgs &a, std::uint32_t cols, std::uint64_t nnz, hipStream_t s) {
+    const int log_split = split_log(a.rows, nnz);
+    const int waves = log_split <= 2 ? 4 : 1 << log_split;
+    const std::uint32_t rows_per_block = static_cast<std::uint32_t>(waves >> log_split);
+    const std::uint64_t bytes = cols != 0u ? ((cols - 1u) * static_cast<std::uint64_t>(a.rhs_ld) + kN) * sizeof(RhsT) : 0u;
+    hipLaunchKernelGGL((qcsr_bwd_values_split<RhsT, kN>), dim3((a.rows + rows_per_block - 1u) / rows_per_block),
+                       dim3(waves * kWave), 0, s, a, log_split, cols, static_cast<std::uint32_t>(bytes));
+}
+
 // Any N / alignment: lanes over the row's entries, columns in order (grad_Y row read
 // uniformly by the wave).
 template<typename RhsT>
@@ -124,11 +215,28 @@ __global__ __launch_bounds__(kWave *kWavesPerBlock) void qcsr_bwd_values_generic
     }
 }
 
+// Entries up to which the gathers (the split rows, or the general form where N is 192 or 256) beat
+// the gene parts. Times in us, split / parts, by rows (33,538 genes of 1,500 per row; 33,538 of
+// 300; 4,000 of 300):
+//   N = 64:     250: 11 / 461, 9 / 211, 9 / 100;      30,000: 459 / 791, 75 / 298, 70 / 168;
+//            60,000: 892 / 1,231, 142 / 392, 134 / 251; 120,000: 1,510 / 1,340, 302 / 571, 294 / 271
+//   N = 128: 30,000: 746 / 1,753, 128 / 633, 115 / 346; 120,000: 2,513 / 2,945, 502 / 1,361, 473 / 580
+// (the parts take each 64-column block in a launch of its own).
+std::uint64_t bwd_parts_line(std::uint32_t cols, std::int64_t n) {
+    return (15'000'000u + (cols + 1023ull) / 1024u * 4'000'000u) * static_cast<std::uint64_t>(n / 64);
+}
+
 template<typename RhsT>
-int launch_bwd_values(const BwdValuesArgs &a, std::int64_t n, bool aligned, hipStream_t s) {
+int launch_bwd_values(const BwdValuesArgs &a, std::int64_t n, bool aligned, std::uint32_t cols, std::uint64_t nnz,
+                      hipStream_t s) {
     const dim3 grid((a.rows + kWavesPerBlock - 1) / kWavesPerBlock), block(kWave * kWavesPerBlock);
     constexpr bool kHalf = sizeof(RhsT) == 2;
-    if (aligned && n == 64) {
+    constexpr int kFirst = kHalf ? 64 : 32;  // 8 lanes per entry; twice that, 16
+    if (aligned && n == kFirst && split_range(cols, a.rhs_ld, sizeof(RhsT), n)) {
+        launch_bwd_split<RhsT, kFirst>(a, cols, nnz, s);
+    } else if (aligned && n == 2 * kFirst && split_range(cols, a.rhs_ld, sizeof(RhsT), n)) {
+        launch_bwd_split<RhsT, 2 * kFirst>(a, cols, nnz, s);
+    } else if (aligned && n == 64) {
         hipLaunchKernelGGL((qcsr_bwd_values_rowwave<RhsT, 64>), grid, block, 0, s, a);
     } else if (aligned && n == 128) {
         hipLaunchKernelGGL((qcsr_bwd_values_rowwave<RhsT, 128>), grid, block, 0, s, a);
@@ -408,11 +516,13 @@ extern "C" int cx_qcsr_spmm_bwd_values(const cx_qcsr_matrix *m, const float *gra
     const bool aligned = aligned16(grad_out) && aligned16(rhs) && (grad_out_ld * 4) % 16 == 0
         && (rhs_ld * static_cast<std::int64_t>(esize)) % 16 == 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (bwd_values_parts_applicable(m->rows, m->cols, rhs_dtype, out_cols, aligned, rhs_ld))
-        return launch_bwd_values_parts(m->row_ptr, m->col_idx, grad_out, grad_out_ld, rhs, rhs_ld, grad_values,
+    if (bwd_values_parts_applicable(m->rows, m->cols, rhs_dtype, out_cols, aligned, rhs_ld)
+        && (m->nnz >= bwd_parts_line(m->cols, out_cols)
+            || (out_cols == 64 && !split_range(m->cols, rhs_ld, sizeof(std::uint16_t), out_cols))))
+        return launch_bwd_values_parts(m->row_ptr, m->col_idx, grad_out, grad_out_ld, rhs, rhs_ld, out_cols, grad_values,
                                        m->rows, m->cols, (m->flags & CX_QCSR_COLUMNS_SORTED) != 0u, s);
-    if (rhs_dtype == CELLERATOR_DTYPE_F16) return launch_bwd_values<std::uint16_t>(a, out_cols, aligned, s);
-    return launch_bwd_values<float>(a, out_cols, aligned, s);
+    if (rhs_dtype == CELLERATOR_DTYPE_F16) return launch_bwd_values<std::uint16_t>(a, out_cols, aligned, m->cols, m->nnz, s);
+    return launch_bwd_values<float>(a, out_cols, aligned, m->cols, m->nnz, s);
 }
 
 extern "C" int cx_qcsr_spmm_bwd_rhs(const cx_qcsr_matrix *transposed, const float *grad_out,

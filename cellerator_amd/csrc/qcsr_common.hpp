@@ -3,6 +3,8 @@
 
 #include "cx_common.hpp"
 
+#include <type_traits>
+
 namespace cx {
 
 enum class ValueMode : int { quantized = 0, f16 = 1, f32 = 2 };
@@ -149,11 +151,24 @@ bool csr_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint64_t 
 std::uint64_t csr_parts_bytes(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz);
 int launch_csr_parts(const cx_qcsr_matrix &m, const float *g, std::int64_t g_ld, std::int64_t n, float *out,
                      std::int64_t out_ld, void *workspace, hipStream_t stream);
-// grad_values of the backward pass by gene part (fp16 weights, N = 64).
+// Weight gathers through one descriptor over [cols x n] (qcsr_spmm_split, qcsr_bwd_values_split):
+// the byte offset of an entry that reads as 0, past every range, and whether a range fits.
+constexpr std::uint32_t kNoEntry = 0x7fff8000u;
+inline bool split_range(std::uint32_t cols, std::int64_t rhs_ld, std::size_t esize, std::int64_t n) {
+    return static_cast<std::uint64_t>(cols) * static_cast<std::uint64_t>(rhs_ld) * esize + n * esize <= 0x7fff0000ull;
+}
+// Waves per row (log2): about 8 waves per SIMD over the chip, and at least one 64-entry chunk per
+// wave.
+inline int split_log(std::uint32_t rows, std::uint64_t nnz) {
+    int l = 0;
+    while (l < 4 && (static_cast<std::uint64_t>(rows) << l) < 8192u && (nnz / rows) >> l > static_cast<std::uint64_t>(kWave)) ++l;
+    return l;
+}
+// grad_values of the backward pass by gene part (fp16 weights, whole 64-column blocks up to 256).
 bool bwd_values_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint32_t rhs_dtype,
                                  std::int64_t out_cols, bool aligned, std::int64_t rhs_ld);
 int launch_bwd_values_parts(const std::int32_t *row_ptr, const std::int32_t *col_idx, const float *grad_out,
-                            std::int64_t grad_out_ld, const void *rhs, std::int64_t rhs_ld,
+                            std::int64_t grad_out_ld, const void *rhs, std::int64_t rhs_ld, std::int64_t out_cols,
                             float *grad_values, std::uint32_t rows, std::uint32_t cols, bool sorted,
                             hipStream_t stream);
 
@@ -165,6 +180,35 @@ __device__ __forceinline__ void set_wave_priority(int p) {
     case 2: __builtin_amdgcn_s_setprio(2); break;
     default: __builtin_amdgcn_s_setprio(3); break;
     }
+}
+
+// Lane j of each group of 8 gets the group's sum of d[j]: 17 instructions for 8 sums (the DPP
+// butterfly of each, and a select to keep it, took 32). First the half-row mirror: lanes 0..3
+// keep d[k], lanes 4..7 (the odd banks, by the write mask) d[k + 4]; then two exchanges within
+// the quad. s_nop: a DPP operand may not be read within two states of a VALU write.
+__device__ __forceinline__ float group_scatter8(float d0, float d1, float d2, float d3, float d4, float d5, float d6,
+                                                float d7, int j) {
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %3, %3, %3 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %0, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %1, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %2, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %3, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xa"
+        : "+v"(d0), "+v"(d1), "+v"(d2), "+v"(d3)
+        : "v"(d4), "v"(d5), "v"(d6), "v"(d7));
+    auto dpp = [](float v, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    using Xor2 = std::integral_constant<int, 0x4E>;
+    using Xor1 = std::integral_constant<int, 0xB1>;
+    const float a0 = d0 + dpp(d0, Xor2{}), a2 = d2 + dpp(d2, Xor2{});
+    const float a1 = d1 + dpp(d1, Xor2{}), a3 = d3 + dpp(d3, Xor2{});
+    const float b0 = (j & 2) != 0 ? a2 : a0, b1 = (j & 2) != 0 ? a3 : a1;
+    const float c0 = b0 + dpp(b0, Xor1{}), c1 = b1 + dpp(b1, Xor1{});
+    return (j & 1) != 0 ? c1 : c0;
 }
 
 __device__ __forceinline__ void wave_sync() {

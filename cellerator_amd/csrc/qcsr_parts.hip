@@ -751,15 +751,8 @@ struct BwdPartsArgs {
     float *grad_values;
     std::uint32_t rows;
     std::uint32_t cols;
+    std::uint32_t add;  // columns of the blocks before this one: add to what they left
 };
-
-// Sum over the 8 lanes of each lane group (quad xor 1, xor 2, then the half-row mirror).
-__device__ __forceinline__ float group_sum8(float d) {
-    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0xB1, 0xf, 0xf, false));
-    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x4E, 0xf, 0xf, false));
-    d += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), 0x141, 0xf, 0xf, false));
-    return d;
-}
 
 template<int kWaves, int kLayers>
 struct BwdGroupsShared {
@@ -772,34 +765,33 @@ struct BwdGroupsShared {
     std::uint32_t rows[kRows];
 };
 
-__device__ __forceinline__ float dot8x2(const float (&g)[8], uint4 w) {
-    float d0 = 0.0f, d1 = 0.0f;
-    d0 = __builtin_fmaf(g[0], h2f(static_cast<std::uint16_t>(w.x & 0xffffu)), d0);
-    d1 = __builtin_fmaf(g[1], h2f(static_cast<std::uint16_t>(w.x >> 16)), d1);
-    d0 = __builtin_fmaf(g[2], h2f(static_cast<std::uint16_t>(w.y & 0xffffu)), d0);
-    d1 = __builtin_fmaf(g[3], h2f(static_cast<std::uint16_t>(w.y >> 16)), d1);
-    d0 = __builtin_fmaf(g[4], h2f(static_cast<std::uint16_t>(w.z & 0xffffu)), d0);
-    d1 = __builtin_fmaf(g[5], h2f(static_cast<std::uint16_t>(w.z >> 16)), d1);
-    d0 = __builtin_fmaf(g[6], h2f(static_cast<std::uint16_t>(w.w & 0xffffu)), d0);
-    d1 = __builtin_fmaf(g[7], h2f(static_cast<std::uint16_t>(w.w >> 16)), d1);
-    return d0 + d1;
+__device__ __forceinline__ float dot8(const float (&g)[8], uint4 w) {
+    float d = g[0] * h2f(static_cast<std::uint16_t>(w.x & 0xffffu));
+    d = __builtin_fmaf(g[1], h2f(static_cast<std::uint16_t>(w.x >> 16)), d);
+    d = __builtin_fmaf(g[2], h2f(static_cast<std::uint16_t>(w.y & 0xffffu)), d);
+    d = __builtin_fmaf(g[3], h2f(static_cast<std::uint16_t>(w.y >> 16)), d);
+    d = __builtin_fmaf(g[4], h2f(static_cast<std::uint16_t>(w.z & 0xffffu)), d);
+    d = __builtin_fmaf(g[5], h2f(static_cast<std::uint16_t>(w.z >> 16)), d);
+    d = __builtin_fmaf(g[6], h2f(static_cast<std::uint16_t>(w.w & 0xffffu)), d);
+    d = __builtin_fmaf(g[7], h2f(static_cast<std::uint16_t>(w.w >> 16)), d);
+    return d;
 }
 
 template<int kWaves, int kLayers, bool kSorted>
 __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPartsArgs a) {
     using Shared = BwdGroupsShared<kWaves, kLayers>;
-    constexpr int kRows = Shared::kRows;
     __shared__ Shared sh;
     const int tid = static_cast<int>(threadIdx.x);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int lane = tid % kWave;
     const int grp = lane >> 3;
     const int j = lane & 7;
-    const std::uint32_t first = blockIdx.x * static_cast<std::uint32_t>(kRows);
-    const std::uint32_t last = first + kRows < a.rows ? first + kRows : a.rows;
+    // an even share of the rows, at most Shared::kRows (as qcsr_spmm_groups)
+    const std::uint32_t first = static_cast<std::uint32_t>(std::uint64_t{blockIdx.x} * a.rows / gridDim.x);
+    const std::uint32_t last = static_cast<std::uint32_t>((std::uint64_t{blockIdx.x} + 1u) * a.rows / gridDim.x);
 
     if (tid < 8) sh.w[kPadGene * 8 + tid] = make_uint4(0u, 0u, 0u, 0u);
-    assign_groups<kWaves, kLayers>(sh.u.pro, sh.rows, a.row_ptr, a.rows, first, tid);
+    assign_groups<kWaves, kLayers>(sh.u.pro, sh.rows, a.row_ptr, last, first, tid);
 
     const int wg_begin = __builtin_amdgcn_readfirstlane(a.row_ptr[first]);
     const int wg_end = __builtin_amdgcn_readfirstlane(a.row_ptr[last]);
@@ -864,6 +856,7 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPart
         __syncthreads();
 #pragma unroll
         for (int l = 0; l < kLayers; ++l) {
+            set_wave_priority(3 - l);  // a wave that is behind issues first (qcsr_spmm_stream)
             for (;;) {
                 if (tail) fix_tail(l);
                 const int nv = end[l] - cur[l] - 8 * j;
@@ -900,41 +893,28 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPart
                     if (f == 1) load_cols(l, 0, e1);
                     if (f == 3) load_cols(l, 1, e1);
                     if (live) {
-                        // stage slot pair `it` holds window entries 8 it + 2f and 8 it + 2f + 1:
-                        // lane it of the group keeps their results in res[2f], res[2f + 1]
-                        const int n2 = (fill_count(rmax, f) + 1) >> 1;
-                        res[2 * f] = res[2 * f + 1] = 0.0f;
-                        int it = 0;
-                        for (; it + 2 <= n2; it += 2) {
-                            const uint4 e = reinterpret_cast<const uint4 *>(sp)[it >> 1];
-                            const uint4 w0 = *reinterpret_cast<const uint4 *>(wbase + e.x);
-                            const uint4 w1 = *reinterpret_cast<const uint4 *>(wbase + e.y);
-                            const uint4 w2 = *reinterpret_cast<const uint4 *>(wbase + e.z);
-                            const uint4 w3 = *reinterpret_cast<const uint4 *>(wbase + e.w);
-                            const float d0 = group_sum8(dot8x2(g[l], w0));
-                            const float d1 = group_sum8(dot8x2(g[l], w1));
-                            const float d2 = group_sum8(dot8x2(g[l], w2));
-                            const float d3 = group_sum8(dot8x2(g[l], w3));
-                            if (j == it) {
-                                res[2 * f] = d0;
-                                res[2 * f + 1] = d1;
-                            }
-                            if (j == it + 1) {
-                                res[2 * f] = d2;
-                                res[2 * f + 1] = d3;
+                        // stage slots 2j and 2j + 1 hold window entries 8j + 2f and 8j + 2f + 1:
+                        // lane j of the group keeps their sums in res[2f], res[2f + 1]
+                        const int cnt = fill_count(rmax, f);
+                        float d[16];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            if (4 * q < cnt) {
+                                const uint4 e = reinterpret_cast<const uint4 *>(sp)[q];
+                                const uint4 w0 = *reinterpret_cast<const uint4 *>(wbase + e.x);
+                                const uint4 w1 = *reinterpret_cast<const uint4 *>(wbase + e.y);
+                                const uint4 w2 = *reinterpret_cast<const uint4 *>(wbase + e.z);
+                                const uint4 w3 = *reinterpret_cast<const uint4 *>(wbase + e.w);
+                                d[4 * q] = dot8(g[l], w0);
+                                d[4 * q + 1] = dot8(g[l], w1);
+                                d[4 * q + 2] = dot8(g[l], w2);
+                                d[4 * q + 3] = dot8(g[l], w3);
+                            } else {
+                                d[4 * q] = d[4 * q + 1] = d[4 * q + 2] = d[4 * q + 3] = 0.0f;
                             }
                         }
-                        if (it < n2) {
-                            const uint2 e = reinterpret_cast<const uint2 *>(sp)[it];
-                            const uint4 w0 = *reinterpret_cast<const uint4 *>(wbase + e.x);
-                            const uint4 w1 = *reinterpret_cast<const uint4 *>(wbase + e.y);
-                            const float d0 = group_sum8(dot8x2(g[l], w0));
-                            const float d1 = group_sum8(dot8x2(g[l], w1));
-                            if (j == it) {
-                                res[2 * f] = d0;
-                                res[2 * f + 1] = d1;
-                            }
-                        }
+                        res[2 * f] = group_scatter8(d[0], d[2], d[4], d[6], d[8], d[10], d[12], d[14], j);
+                        res[2 * f + 1] = group_scatter8(d[1], d[3], d[5], d[7], d[9], d[11], d[13], d[15], j);
                     }
                 }
                 // this lane's window slots in the run: entries cur + 8j .. cur + 8j + in_run - 1
@@ -942,6 +922,15 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPart
                 const std::uint32_t o0 = static_cast<std::uint32_t>(cur[l] + 8 * j) * 4u;
                 if (in_run == 8) {
                     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+                    if (a.add != 0u) {
+                        const u32x4 o0v = __builtin_amdgcn_raw_buffer_load_b128(ro, o0, 0, 0);
+                        const u32x4 o1v = __builtin_amdgcn_raw_buffer_load_b128(ro, o0 + 16u, 0, 0);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            res[k] += __uint_as_float(o0v[k]);
+                            res[4 + k] += __uint_as_float(o1v[k]);
+                        }
+                    }
                     const u32x4 lo4 = {__float_as_uint(res[0]), __float_as_uint(res[1]), __float_as_uint(res[2]),
                                        __float_as_uint(res[3])};
                     const u32x4 hi4 = {__float_as_uint(res[4]), __float_as_uint(res[5]), __float_as_uint(res[6]),
@@ -951,7 +940,12 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPart
                 } else {
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
-                        if (k < in_run) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(res[k]), ro, o0 + 4u * k, 0, 0);
+                        if (k < in_run) {
+                            const float old = a.add != 0u
+                                ? __uint_as_float(static_cast<std::uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(ro, o0 + 4u * k, 0, 0)))
+                                : 0.0f;
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a.add != 0u ? res[k] + old : res[k]), ro, o0 + 4u * k, 0, 0);
+                        }
                 }
                 if constexpr (!kSorted)
                     if (okc != in_run) end[l] = -1;  // broken: no further runs; recomputed at the end
@@ -973,10 +967,15 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_bwd_values_groups(BwdPart
             const int gsel = __builtin_ctzll(todo) >> 3;
             todo &= todo - 1u;
             const std::uint32_t r = sh.rows[(wave * kLayers + l) * 8 + gsel];
-            const float gl = a.grad_out[static_cast<std::int64_t>(r) * a.grad_out_ld + lane];
+            const float *gr = a.grad_out + static_cast<std::int64_t>(r) * a.grad_out_ld + lane;
             for (int i = a.row_ptr[r]; i < a.row_ptr[r + 1]; ++i) {
                 const std::uint32_t col = static_cast<std::uint32_t>(a.col_idx[i]);
-                float d = col < a.cols ? gl * h2f(a.rhs[static_cast<std::int64_t>(col) * a.rhs_ld + lane]) : 0.0f;
+                float d = 0.0f;
+                if (col < a.cols) {
+                    const std::uint16_t *w = a.rhs + static_cast<std::int64_t>(col) * a.rhs_ld + lane;
+                    // with the blocks before this one (the walk may have added to some entries)
+                    for (int c = -static_cast<int>(a.add); c <= 0; c += 64) d = __builtin_fmaf(gr[c], h2f(w[c]), d);
+                }
                 d = xor_reduce<0, 5>(d);
                 if (lane == 0) a.grad_values[i] = d;
             }
@@ -1018,23 +1017,26 @@ bool qcsr_parts_applicable(const QcsrArgs &a, std::uint32_t bits, std::uint32_t 
 // the epilogue's bias and initial values).
 bool bwd_values_parts_applicable(std::uint32_t rows, std::uint32_t cols, std::uint32_t rhs_dtype,
                                  std::int64_t out_cols, bool aligned, std::int64_t rhs_ld) {
-    return rhs_dtype == CELLERATOR_DTYPE_F16 && out_cols == 64 && aligned && rows > 0u && cols > 0u
+    return rhs_dtype == CELLERATOR_DTYPE_F16 && out_cols > 0 && out_cols % 64 == 0 && out_cols <= 256 && aligned && rows > 0u && cols > 0u
         && cols <= static_cast<std::uint32_t>(INT32_MAX) && rhs_ld <= (INT32_MAX / 2) / kPartGenes;
 }
 
 int launch_bwd_values_parts(const std::int32_t *row_ptr, const std::int32_t *col_idx, const float *grad_out,
-                            std::int64_t grad_out_ld, const void *rhs, std::int64_t rhs_ld,
+                            std::int64_t grad_out_ld, const void *rhs, std::int64_t rhs_ld, std::int64_t out_cols,
                             float *grad_values, std::uint32_t rows, std::uint32_t cols, bool sorted,
                             hipStream_t stream) {
     constexpr int kWaves = 16, kLayers = 4;
-    const BwdPartsArgs a{row_ptr, col_idx, grad_out, grad_out_ld, static_cast<const std::uint16_t *>(rhs), rhs_ld,
-                         grad_values, rows, cols};
-    const unsigned rows_per_block = kWaves * kLayers * 8;
-    const dim3 grid((rows + rows_per_block - 1) / rows_per_block), block(kWaves * kWave);
-    if (sorted)
-        hipLaunchKernelGGL((qcsr_bwd_values_groups<kWaves, kLayers, true>), grid, block, 0, stream, a);
-    else
-        hipLaunchKernelGGL((qcsr_bwd_values_groups<kWaves, kLayers, false>), grid, block, 0, stream, a);
+    // one round of the CUs on matrices that full blocks would not fill (100k rows: 196 blocks of
+    // 512 took 1,362 us, 256 of 391 take 1,243)
+    const dim3 grid(round_block_count(rows, kWaves * kLayers * 8, blocks_per_round(), false)), block(kWaves * kWave);
+    for (std::int64_t c0 = 0; c0 < out_cols; c0 += 64) {
+        const BwdPartsArgs a{row_ptr, col_idx, grad_out + c0, grad_out_ld, static_cast<const std::uint16_t *>(rhs) + c0, rhs_ld,
+                             grad_values, rows, cols, static_cast<std::uint32_t>(c0)};
+        if (sorted)
+            hipLaunchKernelGGL((qcsr_bwd_values_groups<kWaves, kLayers, true>), grid, block, 0, stream, a);
+        else
+            hipLaunchKernelGGL((qcsr_bwd_values_groups<kWaves, kLayers, false>), grid, block, 0, stream, a);
+    }
     return check_launch("qcsr_bwd_values_groups");
 }
 

@@ -156,9 +156,6 @@ __global__ __launch_bounds__(kWave *kWavesPerBlock) void qcsr_spmm_rowwave(QcsrA
 
 // ---- split rows: 1 to 16 waves per row ---------------------------------------------------
 
-// Byte offset of a staged entry that reads as 0: past every W range (split_applicable).
-constexpr std::uint32_t kNoEntry = 0x7fff8000u;
-
 // The row-wave form with each row's 64-entry chunks dealt to 2^log_split waves of a workgroup
 // (chunk c to wave c modulo their count) whose sums are added through LDS in wave order. The
 // next chunk's columns and codes load under the current chunk's weight gathers, and W rows are
@@ -274,18 +271,6 @@ __global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int lo
         for (int q = 1; q < (1 << log_split); ++q) v += part[wave + q][c];
         a.out[static_cast<std::int64_t>(row) * a.out_ld + c] = a.ep.active ? epilogue_value(a.ep, v, row, c) : v;
     }
-}
-
-// W read at 32-bit offsets below kNoEntry.
-bool split_applicable(const QcsrArgs &a, std::size_t esize, std::int64_t n) {
-    return static_cast<std::uint64_t>(a.cols) * static_cast<std::uint64_t>(a.rhs_ld) * esize + n * esize <= 0x7fff0000ull;
-}
-
-// Waves per row (log2): about 8 waves per SIMD over the chip, and at least one chunk per wave.
-int split_log(const QcsrArgs &a, std::uint64_t nnz) {
-    int l = 0;
-    while (l < 4 && (static_cast<std::uint64_t>(a.rows) << l) < 8192u && (nnz / a.rows) >> l > kWave) ++l;
-    return l;
 }
 
 template<int kBits, int kPolicy, ValueMode kMode, typename RhsT, int kN>
@@ -440,8 +425,8 @@ int launch_rhs(const QcsrArgs &a, std::int64_t n, bool aligned, const Balance *b
         return launch_balanced<kBits, kPolicy, kMode, RhsT, 64>(a, *bal, stream);
     if (bal != nullptr && aligned && n == 128)
         return launch_balanced<kBits, kPolicy, kMode, RhsT, 128>(a, *bal, stream);
-    if (aligned && (n == 32 || n == 64 || n == 128) && split_applicable(a, sizeof(RhsT), n)) {
-        const int l = split_log(a, nnz);
+    if (aligned && (n == 32 || n == 64 || n == 128) && split_range(a.cols, a.rhs_ld, sizeof(RhsT), n)) {
+        const int l = split_log(a.rows, nnz);
         if (n == 32) launch_split<kBits, kPolicy, kMode, RhsT, 32>(a, l, stream);
         else if (n == 64) launch_split<kBits, kPolicy, kMode, RhsT, 64>(a, l, stream);
         else launch_split<kBits, kPolicy, kMode, RhsT, 128>(a, l, stream);
@@ -504,7 +489,7 @@ bool split_preferred(const QcsrArgs &a, std::uint64_t nnz, std::int64_t n) {
     const std::uint64_t parts = (a.cols + 1023u) / 1024u;
     std::uint64_t line = 30'000'000u + parts * 1'000'000u;
     if (n % 128 == 0) line += line / 2u;
-    return nnz < line && split_applicable(a, sizeof(std::uint16_t), n);
+    return nnz < line && split_range(a.cols, a.rhs_ld, sizeof(std::uint16_t), n);
 }
 
 __global__ void pack_gene_affine_kernel(const float *scales, const float *offsets, std::uint32_t cols,

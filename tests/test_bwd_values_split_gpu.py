@@ -1,0 +1,68 @@
+"""grad_values by gathers with several waves per row (qcsr_bwd_values_split), and by gene part
+in several 64-column blocks (qcsr_bwd_values_groups adding to the block before)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.helpers import check_against_referee, quantized_fixture, to_device_qcsr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,mean,n,dtype", [(1, 1500.0, 64, np.float16), (3, 2500.0, 128, np.float16),
+                                               (50, 65.0, 64, np.float16), (700, 130.0, 128, np.float16),
+                                               (9, 400.0, 32, np.float32), (333, 64.0, 64, np.float32)])
+def test_bwd_values_split(oracle, rows, mean, n, dtype):
+    """One to sixteen waves per row, 8 and 16 lanes per entry, ragged and empty rows; entries
+    outside [0, cols) get 0 even from an infinite row of grad_out."""
+    import torch
+
+    from cellerator_amd import qcsr_spmm_bwd_values
+    rng = np.random.default_rng(rows + n)
+    fx = quantized_fixture(oracle, rng, rows, 3000, mean, 4, 1, empty_every=0 if rows == 1 else 4)
+    g = rng.standard_normal((rows, n)).astype(np.float32)
+    w = (rng.standard_normal((3000, n)) * 0.1).astype(dtype)
+    m, gt, wt = to_device_qcsr(fx), torch.from_numpy(g).cuda(), torch.from_numpy(w).cuda()
+    got = qcsr_spmm_bwd_values(m, gt, wt)
+    ref = oracle.spmm_bwd_values(fx["row_ptr"], fx["col_idx"], g, w)
+    rows_of = np.repeat(np.arange(rows), np.diff(fx["row_ptr"]))
+    mag = np.einsum("ij,ij->i", np.abs(g.astype(np.float64))[rows_of], np.abs(w.astype(np.float64))[fx["col_idx"]])
+    check_against_referee(oracle, ref, mag, got.cpu().numpy())
+    bad = torch.arange(0, m.nnz, 7, device="cuda")
+    col = m.col_idx.clone()
+    col[bad] = torch.tensor([-1, 3000, 2**31 - 1], dtype=torch.int32, device="cuda")[torch.arange(len(bad), device="cuda") % 3]
+    m.col_idx = col
+    gt[-1] = float("inf")
+    again = qcsr_spmm_bwd_values(m, gt, wt)
+    assert (again[bad] == 0).all()
+    keep = torch.ones(m.nnz, dtype=torch.bool, device="cuda")
+    keep[bad] = False
+    keep[int(m.row_ptr[-2]):] = False
+    assert torch.equal(again[keep], got[keep])
+
+
+def test_bwd_values_parts_in_blocks():
+    """N = 192 on a matrix past the line: three blocks, the later ones adding to the first; rows out
+    of order across parts and entries outside the matrix take the per-row path in each block."""
+    import torch
+
+    from cellerator_amd import qcsr_spmm_bwd_values
+    from cellerator_amd.synth import QcsrConfig, dense_normal, generate_qcsr
+    rows, cols, n = 200_003, 1_100, 192
+    m = generate_qcsr(QcsrConfig("blocks", rows, cols, 8, 380.0, 0.2, zipf_s=0.3, nnz_min=40, seed=3))
+    assert m.nnz >= (15_000_000 + 2 * 4_000_000) * 3
+    w, g = dense_normal((cols, n), 0.1, torch.float16, seed=1), dense_normal((rows, n), 1.0, torch.float32, seed=2)
+    rp = m.row_ptr.long()
+    for r in (7, 100_000, rows - 1):  # reversed columns
+        m.col_idx[rp[r]:rp[r + 1]] = m.col_idx[rp[r]:rp[r + 1]].flip(0).clone()
+    m.col_idx[rp[11] + 20] = cols
+    m.col_idx[rp[200] + 1] = -1
+    out = qcsr_spmm_bwd_values(m, g, w)
+    assert float(out[rp[11] + 20]) == 0.0 and float(out[rp[200] + 1]) == 0.0
+    for r in [7, 11, 200, 100_000, rows - 1, *range(500, 520), *range(rows - 40, rows)]:
+        c = m.col_idx[rp[r]:rp[r + 1]].long()
+        ok = (c >= 0) & (c < cols)
+        wr = w.double()[c.clamp(0, cols - 1)]
+        ref, mag = wr @ g[r].double() * ok, wr.abs() @ g[r].double().abs()
+        assert ((out[rp[r]:rp[r + 1]].double() - ref).abs() <= 1e-4 * ref.abs() + 2.0 ** -20 * mag).all(), r
