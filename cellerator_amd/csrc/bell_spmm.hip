@@ -16,8 +16,9 @@
 //     (0xffffffff) are skipped without touching their values;
 //   * row blocks are visited in an XCD-major order so consecutive row blocks of the
 //     schedule share one XCD's L2 (the weight panel is re-read from L2, not HBM).
-// Quantized path (codes of any width, 32x32 blocks, f32 W, N a multiple of 64): fp32 matrix
-// cores, bell_spmm_quant_mfma below.
+// Quantized path (codes of any width, 32x32 blocks, f32 W, N a multiple of 64): bf16 matrix cores
+// on operands cut exactly in three, bell_spmm_quant_split, and fp32 matrix cores on few row
+// blocks and other W layouts, bell_spmm_quant_mfma below.
 // Unquantized values in blocks of 8, 16 or 32 against a row-major W of any type and width run on
 // the fp32 matrix cores, bell_spmm_plain_mfma below.
 // Generic path (any other block size, quantized shapes the above leave out): one wave per row,
@@ -1035,6 +1036,211 @@ __global__ __launch_bounds__(256) void bell_spmm_quant_lds(BellArgs a, std::int6
     }
 }
 
+// ---- the quantized product on the bf16 matrix cores ---------------------------------------
+//
+// Same decoded values and f32 W, each cut exactly into three bf16 parts (8 bits of the mantissa
+// each, by truncation: x = x0 + x1 + x2), and the six products of parts whose weights reach
+// 2^-24 of the whole, x0w0, x0w1, x1w0, x1w1, x0w2, x2w0, on v_mfma_f32_32x32x16_bf16 (exact
+// products, fp32 accumulation). What is left out is below 2^-23 of |x||w|, under the rounding
+// of an fp32 sum; a one-hot W still returns every decoded value bit for bit. Six bf16
+// instructions do the work of 16 fp32 ones of the same size, so the kernel is bound by the
+// vector instructions that cut the operands (11 per two values: 176 per slot and wave for W,
+// 88 for x, 32 for the decode; 24 matrix instructions of 32 cycles beside them) instead of the
+// fp32 matrix cores.
+//
+// An infinity or NaN in W or the metadata would meet a zero part and turn a sum into NaN that is
+// infinite in fp32 products: a wave whose tile holds any value that is not finite walks its
+// slots again on the fp32 instruction.
+//
+// 100k rows of 24 to 64 blocks, 8-bit, N = 256: 572 us, 788 on the fp32 matrix cores; error against
+// 64 bits 6.0e-7, 7.0e-7 there. Taken from 64 row blocks on.
+__device__ __forceinline__ void cut2(float a, float b, std::uint32_t &p0, std::uint32_t &p1, std::uint32_t &p2) {
+    const std::uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    const float ra = a - __uint_as_float(ua & 0xffff0000u), rb = b - __uint_as_float(ub & 0xffff0000u);
+    const std::uint32_t va = __float_as_uint(ra), vb = __float_as_uint(rb);
+    const float sa = ra - __uint_as_float(va & 0xffff0000u), sb = rb - __uint_as_float(vb & 0xffff0000u);
+    p0 = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+    p1 = __builtin_amdgcn_perm(vb, va, 0x07060302u);
+    p2 = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
+}
+
+struct Cut8 {  // 8 consecutive K values of a lane: three operand fragments
+    std::uint32_t p[3][4];
+
+    __device__ __forceinline__ void set(const float (&v)[8]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cut2(v[2 * q], v[2 * q + 1], p[0][q], p[1][q], p[2][q]);
+    }
+    __device__ __forceinline__ cx_bf16x8 part(int k) const {
+        cx_bf16x8 f;
+        __builtin_memcpy(&f, p[k], 16);
+        return f;
+    }
+};
+
+template<int kBits, int kPolicy>
+__global__ __launch_bounds__(256, 4) void bell_spmm_quant_split(BellArgs a, std::int64_t n) {
+    constexpr bool kOffsets = kPolicy == CX_DECODE_PER_GENE_AFFINE;
+    __shared__ __attribute__((aligned(16))) float wtile[4][32 * 64];
+    __shared__ __attribute__((aligned(16))) float wmeta[4][2 * kWave];  // scales at [0, 64), offsets at [64, 128)
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const std::uint32_t row_blocks = (a.rows + 31u) / 32u;
+    const std::uint32_t slot = xcd_major(blockIdx.x, gridDim.x);
+    const std::uint32_t rb = __builtin_amdgcn_readfirstlane(a.rb_order != nullptr ? a.rb_order[slot] : slot);
+    if (rb >= row_blocks) return;
+    const std::uint32_t width = a.ell_cols / 32u;
+    const std::uint32_t *slots = a.block_col_idx + static_cast<std::uint64_t>(rb) * width;
+    const int m = lane % 32;
+    const int h = lane / 32;
+    const std::uint32_t row = rb * 32u + static_cast<std::uint32_t>(m);
+    const std::uint32_t block_rows = min(32u, a.rows - rb * 32u);
+    const rsrc_t rc = make_rsrc(a.packed + static_cast<std::uint64_t>(rb) * 32u * a.row_stride_bytes,
+                                block_rows * a.row_stride_bytes);
+    // lane (m, h)'s codes of K half q: genes 16 q + 8 h .. + 7, kBits bytes
+    const std::uint32_t code_lane = static_cast<std::uint32_t>(m) * a.row_stride_bytes + static_cast<std::uint32_t>(h) * kBits;
+    const float row_offset = kPolicy == CX_DECODE_COLUMN_SCALE_ROW_OFFSET && row < a.rows ? a.row_offsets[row] : 0.0f;
+    const float *w = static_cast<const float *>(a.rhs);
+    const std::uint32_t row_bytes = static_cast<std::uint32_t>(a.rhs_ld) * 4u;
+    float *wt = wtile[wave];
+    float *mt = wmeta[wave];
+
+    for (std::int64_t n0 = static_cast<std::int64_t>(wave) * 64; n0 < n; n0 += 256) {
+        struct Codes {
+            std::uint32_t q[2][2];
+        };
+        auto load_slot = [&](Codes &c, std::uint32_t s, std::uint32_t bc) {
+            const int co = static_cast<int>(code_lane + s * static_cast<std::uint32_t>(kBits) * 4u);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if constexpr (kBits == 8) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b64(rc, co + 16 * q, 0, 0);
+                    c.q[q][0] = v[0];
+                    c.q[q][1] = v[1];
+                } else if constexpr (kBits == 4) {
+                    c.q[q][0] = static_cast<std::uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rc, co + 8 * q, 0, 0));
+                } else if constexpr (kBits == 2) {
+                    c.q[q][0] = static_cast<std::uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rc, co + 4 * q, 0, 0));
+                } else {
+                    c.q[q][0] = static_cast<std::uint8_t>(__builtin_amdgcn_raw_buffer_load_b8(rc, co + 2 * q, 0, 0));
+                }
+            }
+            const std::uint32_t g0 = bc * 32u;
+            const std::uint32_t genes = g0 < a.cols ? min(32u, a.cols - g0) : 0u;
+            const rsrc_t rw = make_rsrc(w + static_cast<std::int64_t>(g0) * a.rhs_ld, genes * row_bytes);
+            const std::uint32_t lane_off = static_cast<std::uint32_t>(lane / 16) * row_bytes
+                + static_cast<std::uint32_t>(n0 + 4 * (lane % 16)) * 4u;
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                load_lds16(rw, reinterpret_cast<uint4 *>(&wt[q * 256]), lane_off + 4u * row_bytes * q, 0u);
+            const rsrc_t rs = make_rsrc(a.scales + g0, genes * 4u);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void)&mt[0], 4, static_cast<std::uint32_t>(m) * 4u, 0, 0, 0);
+            if constexpr (kOffsets) {
+                const rsrc_t ro = make_rsrc(a.offsets + g0, genes * 4u);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(ro, (lds_void)&mt[kWave], 4, static_cast<std::uint32_t>(m) * 4u, 0, 0, 0);
+            }
+        };
+        // the 8 decoded values of K half q; genes past `cols` are 0
+        auto decode = [&](const Codes &c, int q, std::uint32_t bc, float (&x)[8]) {
+            const int g = 16 * q + 8 * h;
+            float s[8], o[8];
+            *reinterpret_cast<float4 *>(&s[0]) = *reinterpret_cast<const float4 *>(&mt[g]);
+            *reinterpret_cast<float4 *>(&s[4]) = *reinterpret_cast<const float4 *>(&mt[g + 4]);
+            if constexpr (kOffsets) {
+                *reinterpret_cast<float4 *>(&o[0]) = *reinterpret_cast<const float4 *>(&mt[kWave + g]);
+                *reinterpret_cast<float4 *>(&o[4]) = *reinterpret_cast<const float4 *>(&mt[kWave + g + 4]);
+            }
+            const bool whole = bc * 32u + 32u <= a.cols;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const std::uint32_t code = (c.q[q][kBits == 8 ? i / 4 : 0] >> (kBits == 8 ? 8 * (i % 4) : kBits * i)) & ((1u << kBits) - 1u);
+                x[i] = __builtin_fmaf(static_cast<float>(code), s[i], kOffsets ? o[i] : row_offset);
+                if (!whole) x[i] = bc * 32u + static_cast<std::uint32_t>(g + i) < a.cols ? x[i] : 0.0f;
+            }
+        };
+        cx_floatx16 acc[2];
+        auto clear = [&] {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+        };
+        auto walk = [&](auto &&products) {
+            for (std::uint32_t base = 0; base < width; base += kWave) {
+                const std::uint32_t cnt = min(static_cast<std::uint32_t>(kWave), width - base);
+                const std::uint32_t sid = static_cast<std::uint32_t>(lane) < cnt ? slots[base + lane] : kInvalidBlock;
+                for (unsigned long long valid = __ballot(sid != kInvalidBlock); valid != 0ull; valid &= valid - 1ull) {
+                    const int s = __builtin_ctzll(valid);
+                    const std::uint32_t bc = static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(sid), s));
+                    Codes c;
+                    load_slot(c, base + static_cast<std::uint32_t>(s), bc);
+                    __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
+                    __builtin_amdgcn_sched_barrier(0);
+                    products(c, bc);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        clear();
+        walk([&](const Codes &c, std::uint32_t bc) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float x[8];
+                decode(c, q, bc, x);
+                Cut8 ca;
+                ca.set(x);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = wt[(16 * q + 8 * h + i) * 64 + 32 * t + m];
+                    Cut8 cb;
+                    cb.set(v);
+                    // the smallest products first
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(2), cb.part(0), acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(0), cb.part(2), acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(1), cb.part(1), acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(1), cb.part(0), acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(0), cb.part(1), acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca.part(0), cb.part(0), acc[t], 0, 0, 0);
+                }
+            }
+        });
+        bool finite = true;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) finite = finite && __builtin_fabsf(acc[t][i]) < __builtin_inff();
+        if (__ballot(!finite) != 0ull) {
+            clear();
+            walk([&](const Codes &c, std::uint32_t bc) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    float x[8];
+                    decode(c, q, bc, x);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {  // K step of 2: genes 16 q + i (h = 0) and 16 q + 8 + i (h = 1)
+                        const float *b = &wt[(16 * q + 8 * h + i) * 64 + m];
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], b[0], acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], b[32], acc[1], 0, 0, 0);
+                    }
+                }
+            });
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const std::int64_t col = n0 + 32 * t + m;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const std::uint32_t r = rb * 32u + 8u * (i / 4) + 4u * static_cast<std::uint32_t>(h) + (i % 4);
+                if (r < a.rows)
+                    a.out[static_cast<std::int64_t>(r) * a.out_ld + col] =
+                        a.ep.active ? epilogue_value(a.ep, acc[t][i], r, col) : acc[t][i];
+            }
+        }
+    }
+}
+
 // ---- unquantized values on the fp32 matrix cores -----------------------------------------
 //
 // Blocks of 8, 16 or 32, values and W of any type, any N (W row-major): every operand is
@@ -1425,7 +1631,9 @@ int bell_spmm_fwd_impl(const cx_bell_matrix *m, const void *rhs, uint32_t rhs_dt
             && (m->decode_policy != CX_DECODE_PER_GENE_AFFINE || m->column_offsets != nullptr);
 #define CX_QBELL_W(B, P)                                                                                 \
     do {                                                                                                 \
-        if (lds_w) hipLaunchKernelGGL((bell_spmm_quant_lds<B, P, 1>), grid, block, 0, s, a, out_cols);       \
+        if (lds_w && (m->rows + 31u) / 32u >= 64u)                                                       \
+            hipLaunchKernelGGL((bell_spmm_quant_split<B, P>), grid, block, 0, s, a, out_cols);           \
+        else if (lds_w) hipLaunchKernelGGL((bell_spmm_quant_lds<B, P, 1>), grid, block, 0, s, a, out_cols);       \
         else hipLaunchKernelGGL((bell_spmm_quant_mfma<B, P>), grid, block, 0, s, a, out_cols);              \
     } while (0)
 #define CX_QBELL(B)                                                                                      \

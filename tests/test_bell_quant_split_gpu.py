@@ -1,0 +1,61 @@
+"""Quantized Blocked-ELL on the bf16 matrix cores with operands cut in three
+(bell_spmm_quant_split, taken from 64 row blocks on)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.helpers import check_against_referee
+from tests.test_bell_gpu import _quantized_bell_32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits,policy,n", [(8, 1, 256), (4, 2, 64), (2, 1, 320), (1, 2, 128), (8, 2, 192), (4, 1, 256)])
+def test_quant_split(oracle, bits, policy, n):
+    """Within the referee's bound, a one-hot W bit for bit, any row-block order, an epilogue, a ragged
+    row block and block column; values that are not finite end where the fp32 form (W off a
+    16-byte boundary) puts them, and the rest is untouched."""
+    import torch
+
+    from cellerator_amd import BellMatrix, Epilogue, bell_spmm
+    rng = np.random.default_rng(bits * 100 + policy * 10 + n)
+    rows, cols, width = 32 * 66 + 11, 32 * 9 + 5, 70 if n == 64 else 6
+    idx, stride, packed, scales, offsets, row_off = _quantized_bell_32(rng, rows, cols, width, bits, policy)
+    t = lambda a: None if a is None else torch.from_numpy(a).cuda()  # noqa: E731
+    kw = dict(bits=bits, policy=policy, row_stride_bytes=stride, packed=packed, scales=scales,
+              offsets=offsets if policy == 1 else None, row_offsets=row_off if policy == 2 else None)
+    m = BellMatrix(rows, cols, 32, width * 32, t(idx.view(np.int32)), bits=bits, decode_policy=policy,
+                   row_stride_bytes=stride, packed_values=t(packed), column_scales=t(scales),
+                   column_offsets=t(offsets) if policy == 1 else None, row_offsets=t(row_off) if policy == 2 else None)
+    rhs = (rng.standard_normal((cols, n)) * 10.0 ** rng.integers(-6, 6, (cols, 1))).astype(np.float32)
+    ref, mag = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, rhs, **kw)
+    out = bell_spmm(m, t(rhs))
+    check_against_referee(oracle, ref, mag, out.cpu().numpy())
+    order = t(rng.permutation((rows + 31) // 32).astype(np.int32))
+    assert torch.equal(bell_spmm(m, t(rhs), row_block_order=order), out)
+    bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
+    assert torch.equal(bell_spmm(m, t(rhs), epilogue=Epilogue(kind=5, bias=bias)), torch.relu(out + bias))
+    # weights near the end of the normal range, whose lower parts are subnormal
+    tiny = (rng.standard_normal((cols, n)) * 2.0 ** -116).astype(np.float32)
+    ref_t, mag_t = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, tiny, **kw)
+    got_t = bell_spmm(m, t(tiny)).cpu().numpy().astype(np.float64)
+    assert (np.abs(got_t - ref_t) <= 2.0 ** -20 * mag_t).all()
+    onehot = np.zeros((cols, n), np.float32)
+    onehot[np.arange(n) % cols, np.arange(n)] = 1.0
+    dec, _ = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, onehot, **kw)
+    assert np.array_equal(bell_spmm(m, t(onehot)).cpu().numpy().astype(np.float64), dec)
+    bad = t(rhs)
+    bad[3, 5], bad[40, 9], bad[cols - 1, n - 1] = float("inf"), float("nan"), -float("inf")
+    # one product per column that may overflow: two of opposite sign have no sum that is the same
+    # in every order (+inf first, or -inf first), and the two forms add in different orders
+    bad[7, 1] = 3.0e38
+    wide = torch.zeros((cols, n + 1), device="cuda")
+    wide[:, 1:] = bad
+    got, want = bell_spmm(m, bad), bell_spmm(m, wide[:, 1:])
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+    far = torch.isfinite(want)
+    far[:, [1, 5, 9, n - 1]] = False
+    check_against_referee(oracle, out.cpu().numpy()[far.cpu().numpy()].astype(np.float64),
+                          mag.reshape(rows, n)[far.cpu().numpy()], got[far].cpu().numpy())
