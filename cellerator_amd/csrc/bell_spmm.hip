@@ -1044,15 +1044,18 @@ __global__ __launch_bounds__(256) void bell_spmm_quant_lds(BellArgs a, std::int6
 // products, fp32 accumulation). What is left out is below 2^-23 of |x||w|, under the rounding
 // of an fp32 sum; a one-hot W still returns every decoded value bit for bit. Six bf16
 // instructions do the work of 16 fp32 ones of the same size, so the kernel is bound by the
-// vector instructions that cut the operands (11 per two values: 176 per slot and wave for W,
+// vector instructions that cut the operands (11 per two values: 176 per slot and wave for W and 32 to scale it,
 // 88 for x, 32 for the decode; 24 matrix instructions of 32 cycles beside them) instead of the
 // fp32 matrix cores.
 //
-// An infinity or NaN in W or the metadata would meet a zero part and turn a sum into NaN that is
-// infinite in fp32 products: a wave whose tile holds any value that is not finite walks its
-// slots again on the fp32 instruction.
+// The matrix cores take subnormal bf16 operands as zero. W is cut times 2^24 (every part of a
+// nonzero float is then normal) and the sums are scaled back; x's parts are normal where the
+// scales and offsets are zero or at least 2^-60, since every x is then a multiple of 2^-83.
+// An infinity or NaN in W or the metadata (or W times 2^24) would meet a zero part and turn a sum
+// into NaN that is infinite in fp32 products. So a wave whose tile holds any value that is not
+// finite, or whose metadata is smaller, walks its slots again on the fp32 instruction.
 //
-// 100k rows of 24 to 64 blocks, 8-bit, N = 256: 572 us, 788 on the fp32 matrix cores; error against
+// 100k rows of 24 to 64 blocks, 8-bit, N = 256: 618 us, 788 on the fp32 matrix cores; error against
 // 64 bits 6.0e-7, 7.0e-7 there. Taken from 64 row blocks on.
 __device__ __forceinline__ void cut2(float a, float b, std::uint32_t &p0, std::uint32_t &p1, std::uint32_t &p2) {
     const std::uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
@@ -1182,7 +1185,11 @@ __global__ __launch_bounds__(256, 4) void bell_spmm_quant_split(BellArgs a, std:
             }
         };
         clear();
+        auto smallness = [](float v) { return (__float_as_uint(v) << 1) - 1u; };  // of |v|; zero: the largest
+        std::uint32_t smallest = kOffsets ? 0xffffffffu : smallness(row_offset);
         walk([&](const Codes &c, std::uint32_t bc) {
+            smallest = min(smallest, smallness(mt[m]));
+            if constexpr (kOffsets) smallest = min(smallest, smallness(mt[kWave + m]));
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 float x[8];
@@ -1193,7 +1200,7 @@ __global__ __launch_bounds__(256, 4) void bell_spmm_quant_split(BellArgs a, std:
                 for (int t = 0; t < 2; ++t) {
                     float v[8];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) v[i] = wt[(16 * q + 8 * h + i) * 64 + 32 * t + m];
+                    for (int i = 0; i < 8; ++i) v[i] = wt[(16 * q + 8 * h + i) * 64 + 32 * t + m] * 0x1p24f;
                     Cut8 cb;
                     cb.set(v);
                     // the smallest products first
@@ -1206,12 +1213,15 @@ __global__ __launch_bounds__(256, 4) void bell_spmm_quant_split(BellArgs a, std:
                 }
             }
         });
-        bool finite = true;
+        bool sound = smallest >= ((127u - 60u) << 24) - 1u;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) finite = finite && __builtin_fabsf(acc[t][i]) < __builtin_inff();
-        if (__ballot(!finite) != 0ull) {
+            for (int i = 0; i < 16; ++i) {
+                sound = sound && __builtin_fabsf(acc[t][i]) < __builtin_inff();
+                acc[t][i] *= 0x1p-24f;
+            }
+        if (__ballot(!sound) != 0ull) {
             clear();
             walk([&](const Codes &c, std::uint32_t bc) {
 #pragma unroll

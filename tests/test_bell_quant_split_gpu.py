@@ -36,11 +36,20 @@ def test_quant_split(oracle, bits, policy, n):
     assert torch.equal(bell_spmm(m, t(rhs), row_block_order=order), out)
     bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
     assert torch.equal(bell_spmm(m, t(rhs), epilogue=Epilogue(kind=5, bias=bias)), torch.relu(out + bias))
-    # weights near the end of the normal range, whose lower parts are subnormal
+    # weights, then metadata, near the end of the normal range: parts that would be subnormal
     tiny = (rng.standard_normal((cols, n)) * 2.0 ** -116).astype(np.float32)
     ref_t, mag_t = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, tiny, **kw)
     got_t = bell_spmm(m, t(tiny)).cpu().numpy().astype(np.float64)
     assert (np.abs(got_t - ref_t) <= 2.0 ** -20 * mag_t).all()
+    low = np.float32(2.0 ** -112)
+    ms = BellMatrix(rows, cols, 32, width * 32, m.block_col_idx, bits=bits, decode_policy=policy, row_stride_bytes=stride,
+                    packed_values=m.packed_values, column_scales=t(scales * low),
+                    column_offsets=t(offsets * low) if policy == 1 else None,
+                    row_offsets=t(row_off * low) if policy == 2 else None)
+    plain = rng.standard_normal((cols, n)).astype(np.float32)
+    ref_s, mag_s = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, plain, **kw)
+    got_s = bell_spmm(ms, t(plain)).cpu().numpy().astype(np.float64) / float(low)
+    assert (np.abs(got_s - ref_s) <= 2.0 ** -20 * mag_s).all()
     onehot = np.zeros((cols, n), np.float32)
     onehot[np.arange(n) % cols, np.arange(n)] = 1.0
     dec, _ = oracle.bell_spmm_referee(rows, cols, 32, width * 32, idx, None, onehot, **kw)
