@@ -165,7 +165,9 @@ template<int kBits, int kPolicy, ValueMode kMode, typename RhsT, int kN>
 __global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int log_split, std::uint32_t rhs_bytes) {
     using S = WaveShape<RhsT, kN>;
     constexpr int kCpl = S::kCpl, kLpe = S::kLpe, kEps = S::kEps;
-    constexpr int kBatch = 4;  // steps whose gathers are in flight together
+    // Steps whose gathers are in flight together: 8 of fp16 rows (45M entries of 33,538 genes,
+    // N = 128: 792 -> 736 us) and 4 where no more are left; 4 of fp32 rows, whose 8 ran slower.
+    constexpr int kBatch = sizeof(RhsT) == 2 ? 8 : 4;
     __shared__ uint2 stage_all[16][kWave];
     __shared__ float part[16][kN];
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -239,19 +241,24 @@ __global__ __launch_bounds__(16 * kWave) void qcsr_spmm_split(QcsrArgs a, int lo
             wave_sync();
             const int count = static_cast<int>(min(end - c0, static_cast<std::uint32_t>(kWave)));
             cur = load_raw(c0 + step);
-            for (int s0 = 0; s0 < count; s0 += kBatch * kEps) {
-                uint2 e[kBatch];
-                float4 w[kBatch];
+            auto steps = [&](int s0, auto batch) {
+                constexpr int kSteps = decltype(batch)::value;
+                uint2 e[kSteps];
+                float4 w[kSteps];
 #pragma unroll
-                for (int q = 0; q < kBatch; ++q) {
+                for (int q = 0; q < kSteps; ++q) {
                     e[q] = stage[s0 + q * kEps + g];
                     const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw, static_cast<int>(e[q].x + j * 16u), 0, 0);
                     w[q] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
                 }
 #pragma unroll
-                for (int q = 0; q < kBatch; ++q)
+                for (int q = 0; q < kSteps; ++q)
                     fma_row<RhsT, kCpl>(acc, __uint_as_float(e[q].y), reinterpret_cast<const RhsT *>(&w[q]));
-            }
+            };
+            int s0 = 0;
+            if constexpr (kBatch > 4 && kBatch * kEps <= kWave)
+                for (; count - s0 > 4 * kEps; s0 += kBatch * kEps) steps(s0, std::integral_constant<int, kBatch>{});
+            for (; s0 < count; s0 += 4 * kEps) steps(s0, std::integral_constant<int, 4>{});
             wave_sync();
         }
         reduce_groups<kLpe, kCpl>(acc);
@@ -477,12 +484,13 @@ int launch_quantized(const QcsrArgs &a, const cx_qcsr_matrix &m, std::uint32_t r
 
 // Where the split rows beat the row groups over LDS gene parts (qcsr_parts.hip), for the shapes
 // both take. The split rows' time is their gathers', about 10 us per million entries for 64
-// output columns and 17 for 128 (the columns and codes are read once); the row groups pay for
+// output columns and 16 for 128 (the columns and codes are read once); the row groups pay for
 // walking every gene part with few rows per workgroup before the entries count. Times in us,
 // split / row groups, by rows (33,538 genes of 1,500 per row; 33,538 of 300; 4,000 of 300):
-//   N = 64:    250: 12 / 359, 11 / 158, 9 / 82;   30,000: 474 / 643, 105 / 223, 80 / 143;
-//           60,000: 1,101 / 996, 204 / 295, 154 / 214;  120,000: 1,829 / 1,049, 331 / 370, 248 / 229
-//   N = 128: 30,000: 845 / 1,284, 174 / 440, 132 / 281; 120,000: 2,982 / 2,079, 536 / 738, 418 / 448
+//   N = 64:     250: 11 / 359, 12 / 158, 11 / 82;      30,000: 430 / 643, 97 / 223, 76 / 143;
+//            60,000: 1,013 / 996, 186 / 295, 143 / 214; 120,000: 1,829 / 1,049, 331 / 370, 248 / 229
+//   N = 128: 30,000: 739 / 1,284, 155 / 440, 121 / 281; 60,000: 1,619 / 1,979, 295 / 585, 232 / 421;
+//            120,000: 2,982 / 2,079, 536 / 738, 418 / 448 (120,000 rows: with four gathers in flight)
 // So the line is drawn at 30 million entries plus one million per gene part, half as far
 // again where the output is whole blocks of 128 columns.
 bool split_preferred(const QcsrArgs &a, std::uint64_t nnz, std::int64_t n) {
