@@ -215,15 +215,18 @@ __global__ __launch_bounds__(kWave *kWavesPerBlock) void qcsr_bwd_values_generic
     }
 }
 
-// Entries up to which the gathers (the split rows, or the general form where N is 192 or 256) beat
-// the gene parts. Times in us, split / parts, by rows (33,538 genes of 1,500 per row; 33,538 of
-// 300; 4,000 of 300):
+// Where the gathers (the split rows, or the general form where N is 192 or 256) beat the gene
+// parts. Times in us, split / parts, by rows (33,538 genes of 1,500 per row; 33,538 of 300; 4,000
+// of 300):
 //   N = 64:     250: 11 / 461, 9 / 211, 9 / 100;      30,000: 459 / 791, 75 / 298, 70 / 168;
 //            60,000: 892 / 1,231, 142 / 392, 134 / 251; 120,000: 1,510 / 1,340, 302 / 571, 294 / 271
 //   N = 128: 30,000: 746 / 1,753, 128 / 633, 115 / 346; 120,000: 2,513 / 2,945, 502 / 1,361, 473 / 580
-// (the parts take each 64-column block in a launch of its own).
-std::uint64_t bwd_parts_line(std::uint32_t cols, std::int64_t n) {
-    return (15'000'000u + (cols + 1023ull) / 1024u * 4'000'000u) * static_cast<std::uint64_t>(n / 64);
+// (the parts take each 64-column block in a launch of its own, the later ones adding). Both are
+// estimated, the walk by group_walk_us; N = 192 and 256 have no split form, and the general one
+// is left only where the walk takes a fraction of 8.4 us per million entries and block.
+bool bwd_gathers_preferred(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz, std::int64_t n) {
+    const double walk = static_cast<double>(n / 64) * group_walk_us(rows, cols, nnz, 9.6, 0.64) * (n > 64 ? 1.1 : 1.0);
+    return static_cast<double>(nnz) * 1e-6 * (n == 128 ? 14.0 : 8.4 * static_cast<double>(n / 64)) < walk;
 }
 
 template<typename RhsT>
@@ -517,7 +520,7 @@ extern "C" int cx_qcsr_spmm_bwd_values(const cx_qcsr_matrix *m, const float *gra
         && (rhs_ld * static_cast<std::int64_t>(esize)) % 16 == 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (bwd_values_parts_applicable(m->rows, m->cols, rhs_dtype, out_cols, aligned, rhs_ld)
-        && (m->nnz >= bwd_parts_line(m->cols, out_cols)
+        && (!bwd_gathers_preferred(m->rows, m->cols, m->nnz, out_cols)
             || (out_cols == 64 && !split_range(m->cols, rhs_ld, sizeof(std::uint16_t), out_cols))))
         return launch_bwd_values_parts(m->row_ptr, m->col_idx, grad_out, grad_out_ld, rhs, rhs_ld, out_cols, grad_values,
                                        m->rows, m->cols, (m->flags & CX_QCSR_COLUMNS_SORTED) != 0u, s);

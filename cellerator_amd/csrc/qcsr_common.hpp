@@ -157,6 +157,17 @@ constexpr std::uint32_t kNoEntry = 0x7fff8000u;
 inline bool split_range(std::uint32_t cols, std::int64_t rhs_ld, std::size_t esize, std::int64_t n) {
     return static_cast<std::uint64_t>(cols) * static_cast<std::uint64_t>(rhs_ld) * esize + n * esize <= 0x7fff0000ull;
 }
+// Time in us of a row-group walk over LDS gene parts (qcsr_spmm_groups, qcsr_bwd_values_groups), 64
+// output columns: every round of 256 workgroups of up to 512 rows walks every part, a fixed
+// cost per part and one per entry of a row; rounds that give the waves one set of 8 rows
+// (32,768 rows) or two take 0.6 and 0.95 of that. Within 15% of the times listed at the two
+// rules that use it.
+inline double group_walk_us(std::uint32_t rows, std::uint32_t cols, std::uint64_t nnz, double part_us, double entry_us) {
+    const double parts = static_cast<double>((static_cast<std::uint64_t>(cols) + 1023u) / 1024u);
+    const double rounds = static_cast<double>((static_cast<std::uint64_t>(rows) + 131071u) / 131072u);
+    const double fill = rows <= 32768u ? 0.6 : rows <= 65536u ? 0.95 : 1.0;
+    return 60.0 + rounds * fill * (part_us * parts + entry_us * static_cast<double>(nnz) / rows);
+}
 // Waves per row (log2): about 8 waves per SIMD over the chip, and at least one 64-entry chunk per
 // wave.
 inline int split_log(std::uint32_t rows, std::uint64_t nnz) {

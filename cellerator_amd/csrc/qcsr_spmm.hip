@@ -21,7 +21,7 @@
 // qcsr_spmm_split is that form for every plain launch (a row to 1 .. 16 waves, so a few hundred
 // cells fill the chip); qcsr_spmm_rowwave stays for weights past its 2 GiB descriptor and the
 // load-balanced form cuts equal entry ranges. Quantized codes with fp16 weights at N = 64 .. 256
-// leave for the row groups of qcsr_parts.hip above split_preferred's line.
+// leave for the row groups of qcsr_parts.hip where split_preferred finds them faster.
 // Any other shape (N not 32/64/128, unaligned operands) takes the generic kernel: one
 // wave per row, lanes over output columns, entries in nnz order.
 #include "qcsr_common.hpp"
@@ -491,13 +491,15 @@ int launch_quantized(const QcsrArgs &a, const cx_qcsr_matrix &m, std::uint32_t r
 //            60,000: 1,013 / 996, 186 / 295, 143 / 214; 120,000: 1,829 / 1,049, 331 / 370, 248 / 229
 //   N = 128: 30,000: 739 / 1,284, 155 / 440, 121 / 281; 60,000: 1,619 / 1,979, 295 / 585, 232 / 421;
 //            120,000: 2,982 / 2,079, 536 / 738, 418 / 448 (120,000 rows: with four gathers in flight)
-// So the line is drawn at 30 million entries plus one million per gene part, half as far
-// again where the output is whole blocks of 128 columns.
+// So both are estimated: the gathers per entry, the walk by group_walk_us. Rows whose runs fit the
+// walk's 64-entry window (fewer than 40 entries per part on average) cost it less: 70,569 rows of
+// 906 over 29 parts, N = 128, take 775 us where the gathers take 1,015. The walk keeps what is within
+// a tenth.
 bool split_preferred(const QcsrArgs &a, std::uint64_t nnz, std::int64_t n) {
-    const std::uint64_t parts = (a.cols + 1023u) / 1024u;
-    std::uint64_t line = 30'000'000u + parts * 1'000'000u;
-    if (n % 128 == 0) line += line / 2u;
-    return nnz < line && split_range(a.cols, a.rhs_ld, sizeof(std::uint16_t), n);
+    const bool short_runs = nnz < 40ull * a.rows * ((a.cols + 1023ull) / 1024u);
+    const double walk = static_cast<double>(n / 64) * group_walk_us(a.rows, a.cols, nnz, 4.5, short_runs ? 0.30 : 0.53);
+    const double gathers = static_cast<double>(nnz) * 1e-6 * (16.0 * static_cast<double>(n / 128) + (n % 128 != 0 ? 10.0 : 0.0));
+    return gathers < 0.9 * walk && split_range(a.cols, a.rhs_ld, sizeof(std::uint16_t), n);
 }
 
 __global__ void pack_gene_affine_kernel(const float *scales, const float *offsets, std::uint32_t cols,

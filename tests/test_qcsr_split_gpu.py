@@ -48,16 +48,18 @@ def test_split_rows(oracle, bits, policy, rows, mean, n, dtype):
 
 @pytest.mark.parametrize("bits,policy,n", [(4, 3, 64), (8, 1, 64), (2, 2, 128)])
 def test_row_groups_above_the_line(bits, policy, n):
-    """A matrix past split_preferred's line runs on the row groups: a sample of rows from every
-    part of it against float64 (the bound of tests/helpers.py)."""
+    """A matrix large enough for split_preferred to choose the row groups (the gathers' estimate,
+    10 and 16 us per million entries, past the walk's): a sample of rows from every part of it
+    against float64 (the bound of tests/helpers.py)."""
     import torch
 
     from cellerator_amd import QcsrMatrix, qcsr_check_columns, qcsr_pack_gene_affine, qcsr_spmm
     from cellerator_amd import _native as N
     from cellerator_amd.synth import QcsrConfig, dense_normal, generate_qcsr
-    rows, cols = 72_000, 6_000
+    rows, cols = 72_000 if n == 64 else 110_000, 6_000
     m = generate_qcsr(QcsrConfig("line", rows, cols, bits, 1_000.0, 0.4, zipf_s=0.6, seed=5 + bits))
-    assert m.nnz > (30_000_000 + 6_000_000) * (1.5 if n == 128 else 1.0)
+    walk = (n // 64) * (60 + 4.5 * 6 + 0.53 * m.nnz / rows)
+    assert m.nnz * 1e-6 * (16.0 if n == 128 else 10.0) > 0.9 * walk
     w = dense_normal((cols, n), 0.02, torch.float16, seed=3)
     if policy == 2:
         m = QcsrMatrix(rows, cols, bits, m.row_ptr, m.col_idx, packed_row_ptr=m.packed_row_ptr,
