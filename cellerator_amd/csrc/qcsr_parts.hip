@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_spmm_groups(QcsrArgs a) {
     const char *mbase = reinterpret_cast<const char *>(sh.meta);
     uint4 *sp = &sh.u.stage[wave][grp][0];
 
-    const bool rounds = gridDim.x > 256u;  // more than one workgroup per CU, one after the other
+    const bool rounds = gridDim.x > 512u;  // more than two workgroups per CU, one after the other
     const int cols = static_cast<int>(a.cols);
     const int parts = (cols + kPartGenes - 1) / kPartGenes;
     for (int part = static_cast<int>(a.first_part); part < parts; ++part) {
@@ -418,8 +418,9 @@ __global__ __launch_bounds__(kWaves * kWave) void qcsr_spmm_groups(QcsrArgs a) {
         __syncthreads();
 #pragma unroll
         for (int l = 0; l < kLayers; ++l) {
-            // a wave that is behind issues first (qcsr_spmm_stream): 1M rows 6,600 -> 6,340 us, 250k
-            // 1,912 -> 1,873; in a single round, where the longest set decides, 1.5% slower
+            // a wave that is behind issues first (qcsr_spmm_stream): 1M rows 6,600 -> 6,340 us, 500k
+            // 3,515 -> 3,420; two rounds (250k) 3.7% faster on one box and 1.3% slower on another, a
+            // single round, where the longest set decides, 1.5% slower
             if (rounds) set_wave_priority(3 - l);
             for (;;) {
                 if (tail) fix_tail(l);

@@ -154,10 +154,11 @@ typedef struct cx_qcsr_matrix {
 
 /* Y[rows x out_cols] (fp32, row stride out_ld) = decode(A) . RHS[cols x out_cols]
  * (row stride rhs_ld, dtype F16 or F32; F16 widens exactly). fp32 multiply and
- * fp32 accumulation, deterministic (fixed per-row summation order). Quantized codes with
- * F16 RHS at out_cols = 64, 128, 192 or 256 stream RHS through LDS by gene part, 64 output
- * columns per launch: fastest with each row's columns ascending; rows out of order across parts are
- * recomputed per row, and columns outside [0, cols) contribute nothing on that path.
+ * fp32 accumulation, deterministic (fixed per-row summation order for a given shape and entry
+ * count). Quantized codes with F16 RHS at out_cols = 64, 128, 192 or 256 on larger matrices stream
+ * RHS through LDS by gene part, 64 output columns per launch: fastest with each row's columns
+ * ascending; rows out of order across parts are recomputed per row. There, and on smaller matrices
+ * (RHS rows gathered, several waves per row), columns outside [0, cols) contribute nothing.
  * Replaces csr_spmm_fwd_f16_f32 (src/compute/sparse/project/project.hh:12-23). */
 int cx_qcsr_spmm_fwd(const cx_qcsr_matrix *a, const void *rhs, uint32_t rhs_dtype,
                      int64_t rhs_ld, int64_t out_cols, float *out, int64_t out_ld,
@@ -532,8 +533,9 @@ int cx_bell_block_major_values(const cx_bell_matrix *a, void *out, uint64_t capa
                                void *stream);
 
 /* Y = X_bell . RHS with a row-major RHS (F32, F16 or BF16), any block size and N, plain
- * (BF16/F16/F32) or quantized values: fp32 accumulation in slot order per output
- * element, the semantics of blocked_ell_spmm_fwd_kernel_ / quantized_blocked_ell_spmm_fwd_kernel_
+ * (BF16/F16/F32) or quantized values: fp32 products and accumulation in a fixed order per output
+ * element (matrix cores for blocks of 8, 16 and 32 and for quantized 32 x 32; slot order
+ * elsewhere), the semantics of blocked_ell_spmm_fwd_kernel_ / quantized_blocked_ell_spmm_fwd_kernel_
  * (src/compute/sparse/project/kernels/blocked_ell_spmm_fwd_kernel_.cuh:1-33,
  *  quantized_blocked_ell_spmm_fwd_kernel_.cuh:1-39). Replaces
  * blocked_ell_spmm_fwd_f16_f32 / quantized_blocked_ell_spmm_fwd_f32
